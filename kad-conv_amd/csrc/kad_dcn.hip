@@ -1,5 +1,5 @@
-// Modulated deformable 3x3 convolution (DCNv2) fused into an MFMA GEMM, and the
-// plain 3x3 convolution that produces its offsets.
+// The deformable convolutions' entry points (kad_dcn_fwd, kad_dsc_fwd, kad_dsc_fwd_group), the narrow
+// deformable kernel, the plain 3x3 convolution, and the packing of their weights.
 //
 // Semantics: torchvision.ops.deform_conv2d as called by DSC.forward
 // (KAD-Conv/kadconv/kad_conv.py:63-67), one offset group; sampling rule as
@@ -11,45 +11,17 @@
 // 270-300) are fused here too, with deterministic partials instead of float
 // atomics.
 //
-// GEMM view: out[p, co] = sum_k S[p, k] * Wt[k, co] with k = (chunk, tap, c32),
-// M = output pixels, N = Cout, K = 9 * roundup(Cin, 32).
-//
-// One kernel template, three modes:
-//  EXT    offsets (and mask) come from memory             -> kad_dcn_fwd
-//  FUSED  offsets = conv_offset(x) computed in the block   -> kad_dsc_fwd
-//  PLAIN  ordinary 3x3 convolution (no sampling)          -> kad_conv3x3_fwd
-//
-// Block = 512 threads (8 waves, two per SIMD, so one wave's LDS / memory waits
-// overlap the other's MFMA and blend work) x one output tile of up to 128
-// pixels (TH x TW, chosen per image size to waste few lanes) x 16 * NBF output
-// channels; wave w owns tile pixels [16 w, 16 w + 16) and all the block's
-// channels.
-//  0. Loads that do not depend on anything are issued first: epilogue
-//     parameters, the mask (and offsets in EXT mode), the first input chunk.
-//  1. PLAIN / FUSED: the tile's 3x3 footprint (tile + 1-pixel ring, zero
-//     padded) is staged per 32-channel chunk in LDS and convolved on MFMA
-//     (integer taps need no sample records).  FUSED keeps the 18 offset
-//     channels in LDS; PLAIN goes straight to the epilogue.
-//  2. Every (tap, pixel) sample position is computed once (registers), and the
-//     block reduces the bounding box of all live corners.  The input region =
-//     that box, capped to the LDS budget around the tile (typical offsets fit).
-//     Each sample's four region byte offsets and weights (bilinear x mask, 0
-//     for out-of-image corners; fp16 except on the fp32 path) go to LDS once.
-//     Samples outside a capped region are flagged and added by a rare pass
-//     that reads global memory.
-//  3. Per 32-channel chunk (next chunk prefetched into registers): the region
-//     slice [pixels][32 ch] and, on 16-bit paths, the chunk's weights
-//     [9 taps][cols][32] are staged in LDS; for each tap each lane builds its
-//     MFMA A fragment (8 channels of one (pixel, tap)) from four 16-byte LDS
-//     corner reads blended with packed FMAs, and the wave issues NBF
-//     v_mfma_f32_16x16x32 against 16-byte B fragments.  Weight rows are
-//     64 bytes, so their four 16-byte pieces are stored XOR-swizzled by
-//     column (piece g of column c at slot g ^ ((c >> 1) & 3)): the 16 lanes
-//     of a B read then hit distinct banks.
-//  4. Epilogue: bias, BN scale/shift, ReLU, branch scale; the tile is staged
-//     in LDS and written with 16-byte row-contiguous stores; GAP partials.
-// Blocks are mapped so that each XCD (and its L2) gets a contiguous band of
-// tiles: neighbouring tiles share their halos through that L2.
+// Modes: EXT    offsets (and mask) come from memory             -> kad_dcn_fwd
+//        FUSED  offsets = conv_offset(x) computed in the block   -> kad_dsc_fwd
+//        PLAIN  ordinary 3x3 convolution (no sampling)          -> kad_conv3x3_fwd, kad_conv_fwd
+// EXT and FUSED run on kad_dcn_gather.h's kernel, at 16-bit Cout <= 16 on dsc2_kernel below; PLAIN on
+// plain_kernel: block = 512 threads (8 waves) x one output tile of up to 128 pixels (TH x TW, chosen
+// per image size to waste few lanes) x 16 NBF output channels; wave w owns tile pixels [16 w, 16 w + 16)
+// and all the block's channels.  Per 32-channel chunk the tile's 3x3 footprint (tile + 1-pixel ring, zero
+// padded) and, on 16-bit paths, the chunk's weights [9 taps][cols][32] are staged in LDS, the next chunk
+// prefetched into registers.  Weight rows are 64 bytes, so their four 16-byte pieces are stored
+// XOR-swizzled by column (piece g of column c at slot g ^ ((c >> 1) & 3)).  Epilogue: bias, BN
+// scale/shift, activation; the tile is staged in LDS and written with row-contiguous stores.
 //
 // Any consistent assignment of k to (lane group, slot) gives the same dot
 // product, so A and B only have to agree with each other; the accumulator
@@ -58,7 +30,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "kad_common.h"
+#include "kad_dcn.h"
 
 namespace kad {
 
@@ -68,251 +40,27 @@ namespace kad {
 constexpr int DCN_WAVES = KAD_DCN_WAVES;           // waves per block (8: two per SIMD)
 constexpr int DCN_THREADS = 64 * DCN_WAVES;
 constexpr int DCN_WM = 8 / DCN_WAVES;              // 16-pixel A fragments per wave
-constexpr int DCN_TILE = DCN_WAVES * DCN_WM * 16;  // 128 pixels per block
-constexpr int DCN_NPAIR = 9 * DCN_TILE;            // (tap, pixel) samples per block
-constexpr int DCN_KSTEP = DCN_THREADS / DCN_TILE;  // sample (tap, pixel) of thread t: pixel t % 128, taps t / 128 + KSTEP u
-constexpr int DCN_PPT = (9 + DCN_KSTEP - 1) / DCN_KSTEP;  // samples per thread
-constexpr int DCN_NOFF = 18;                       // offset channels (2 x 9 taps)
+static_assert(DCN_WAVES * DCN_WM * 16 == DCN_TILE, "128 pixels per block");
 constexpr int DCN_LDS = 160 * 1024;                // gfx950 LDS per CU
 constexpr int DCN_SLOT = DCN_THREADS / 4;          // region pixels staged per round (4 threads per pixel)
 constexpr int DCN_FCAP = 704;                      // footprint pixels (enough for stride <= 2)
 static_assert(DCN_TILE == 128 && DCN_SLOT % 64 == 0, "tile / staging geometry");
-constexpr int DCN_SE_LDS = 48 * 1024;              // fused SE scratch (floats in the region buffer) limit
 
-enum { MODE_EXT = 0, MODE_FUSED = 1, MODE_PLAIN = 2 };
-
-struct DcnGeom {
-  int ho, wo, th, tw, tiles_x, tiles, grid_x, nchunk, cout_pad;
-  int fh, fw;        // 3x3 footprint of a tile: (th - 1) * stride + 3 rows, likewise columns
-  float inv_tw, inv_fw;
-};
-
-// Tile shape for an Ho x Wo output: TH x TW <= 128 pixels minimising the
-// padded pixel count; ties prefer squarer tiles (smaller halo).
-static void pick_tile(int ho, int wo, int* th_out, int* tw_out) {
-  long best = -1;
-  int bth = 8, btw = 16;
-  for (int tw = 4; tw <= 64; ++tw) {
-    const int th = DCN_TILE / tw;
-    if (th < 1) break;
-    const long cost = (long)ceil_div(ho, th) * ceil_div(wo, tw) * DCN_TILE * 64 + (th > tw ? th - tw : tw - th);
-    if (best < 0 || cost < best) {
-      best = cost;
-      bth = th;
-      btw = tw;
-    }
-  }
-  *th_out = bth;
-  *tw_out = btw;
-}
-
-// ---- sample info ----------------------------------------------------------------------------
-// Fast-path record per (tap, pixel): byte offsets of the four corners inside the
-// staged region and the corner weights (16-bit paths: 16-bit offsets, fp16
-// weights; fp32 path: 32-bit offsets, fp32 weights).  Samples that are dead
-// (all weights 0) or outside a capped region get zero weights here; the latter
-// are accumulated by a separate pass from global memory (s_slow).
-struct __align__(16) Info16 { unsigned o01, o23; unsigned w01, w23; };  // weights as 2 x half2
-struct __align__(16) Info32 { unsigned o[4]; float w[4]; };
-
-__device__ __forceinline__ unsigned pack_h2(float a, float b) {
-  const half2_t h{(half_t)a, (half_t)b};
-  return __builtin_bit_cast(unsigned, h);
-}
-
-template <typename T> struct InfoOf { typedef Info16 type; };
-template <> struct InfoOf<float> { typedef Info32 type; };
-
-template <typename T>
-__device__ __forceinline__ typename InfoOf<T>::type make_info(const unsigned* o, const float* w) {
-  typename InfoOf<T>::type r;
-  if constexpr (sizeof(T) == 4) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      r.o[i] = o[i];
-      r.w[i] = w[i];
-    }
-  } else {
-    r.o01 = o[0] | (o[1] << 16);
-    r.o23 = o[2] | (o[3] << 16);
-    r.w01 = pack_h2(w[0], w[1]);
-    r.w23 = pack_h2(w[2], w[3]);
-  }
-  return r;
-}
-
-// byte offset of corner j of a record
-__device__ __forceinline__ unsigned corner(const Info16& in, int j) {
-  const unsigned v = j < 2 ? in.o01 : in.o23;
-  return (j & 1) ? v >> 16 : v & 0xffffu;
-}
-__device__ __forceinline__ unsigned corner(const Info32& in, int j) { return in.o[j]; }
-
-// ---- A fragment from four corners ------------------------------------------------------------
-template <typename T> struct DcnFrag;
-
-template <> struct DcnFrag<half_t> {
-  typedef half8_t frag;
-  static __device__ __forceinline__ frag blend(const half8_t& v0, const half8_t& v1, const half8_t& v2,
-                                               const half8_t& v3, const Info16& in) {
-    const half2_t w01 = __builtin_bit_cast(half2_t, in.w01), w23 = __builtin_bit_cast(half2_t, in.w23);
-    frag r = v0 * w01[0];
-    r += v1 * w01[1];
-    r += v2 * w23[0];
-    r += v3 * w23[1];
-    return r;
-  }
-  static __device__ __forceinline__ floatx4 mma(const frag& a, const frag& b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
-  }
-};
-
-template <> struct DcnFrag<bf16_t> {
-  typedef bf16x8_t frag;
-  static __device__ __forceinline__ frag blend(const bf16x8_t& v0, const bf16x8_t& v1, const bf16x8_t& v2,
-                                               const bf16x8_t& v3, const Info16& in) {
-    const half2_t w01 = __builtin_bit_cast(half2_t, in.w01), w23 = __builtin_bit_cast(half2_t, in.w23);
-    const float a = (float)w01[0], b = (float)w01[1], c = (float)w23[0], d = (float)w23[1];
-    frag r;
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-      r[j] = (bf16_t)(a * (float)v0[j] + b * (float)v1[j] + c * (float)v2[j] + d * (float)v3[j]);
-    return r;
-  }
-  static __device__ __forceinline__ floatx4 mma(const frag& a, const frag& b, floatx4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-  }
-};
-
-struct f32x8 { floatx4 lo, hi; };
-
-template <> struct DcnFrag<float> {
-  typedef f32x8 frag;
-  static __device__ __forceinline__ frag blend(const f32x8& v0, const f32x8& v1, const f32x8& v2,
-                                               const f32x8& v3, const Info32& in) {
-    frag r;
-    r.lo = v0.lo * in.w[0] + v1.lo * in.w[1] + v2.lo * in.w[2] + v3.lo * in.w[3];
-    r.hi = v0.hi * in.w[0] + v1.hi * in.w[1] + v2.hi * in.w[2] + v3.hi * in.w[3];
-    return r;
-  }
-  // 8 MFMA steps of k=4: step j consumes slot j of every lane group, i.e.
-  // k = 8 * group + j on both operands.
-  static __device__ __forceinline__ floatx4 mma(const frag& a, const frag& b, floatx4 c) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.lo[j], b.lo[j], c, 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a.hi[j], b.hi[j], c, 0, 0, 0);
-    return c;
-  }
-};
-
-template <typename T>
-__device__ __forceinline__ typename DcnFrag<T>::frag ld8(const T* p) {
-  typedef typename DcnFrag<T>::frag F;
-  if constexpr (sizeof(T) == 4) {
-    F r;
-    r.lo = *(const floatx4*)p;
-    r.hi = *(const floatx4*)(p + 4);
-    return r;
-  } else {
-    return *(const F*)p;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ void st8(T* p, const typename DcnFrag<T>::frag& v) {
-  if constexpr (sizeof(T) == 4) {
-    *(floatx4*)p = v.lo;
-    *(floatx4*)(p + 4) = v.hi;
-  } else {
-    *(typename DcnFrag<T>::frag*)p = v;
-  }
-}
-
-template <typename T>
-__device__ __forceinline__ typename DcnFrag<T>::frag zero8() {
-  typedef typename DcnFrag<T>::frag F;
-  if constexpr (sizeof(T) == 4) {
-    F r;
-    r.lo = floatx4{0.f, 0.f, 0.f, 0.f};
-    r.hi = r.lo;
-    return r;
-  } else {
-    return F{};
-  }
-}
-
-// Bilinear geometry of one sample at (py, px) (torchvision's rule): clamped
-// top-left corner, corner steps (0 or 1 per axis) and the four weights times m;
-// all weights 0 for a dead sample.
-__device__ __forceinline__ void sample_geom(float py, float px, float m, int h, int w, int& cy0, int& cx0, int& sy,
-                                            int& sx, float* wt) {
-  cy0 = cx0 = sy = sx = 0;
-  wt[0] = wt[1] = wt[2] = wt[3] = 0.f;
-  if (py > -1.f && py < (float)h && px > -1.f && px < (float)w) {
-    const float fy = floorf(py), fx = floorf(px);
-    const int y0 = (int)fy, x0 = (int)fx, y1 = y0 + 1, x1 = x0 + 1;
-    const float ly = py - fy, lx = px - fx, hy = 1.f - ly, hx = 1.f - lx;
-    const bool vy0 = y0 >= 0, vy1 = y1 <= h - 1, vx0 = x0 >= 0, vx1 = x1 <= w - 1;
-    cy0 = vy0 ? y0 : 0;
-    const int cy1 = vy1 ? y1 : h - 1;
-    cx0 = vx0 ? x0 : 0;
-    const int cx1 = vx1 ? x1 : w - 1;
-    sy = cy1 - cy0;
-    sx = cx1 - cx0;
-    wt[0] = (vy0 && vx0) ? hy * hx * m : 0.f;
-    wt[1] = (vy0 && vx1) ? hy * lx * m : 0.f;
-    wt[2] = (vy1 && vx0) ? ly * hx * m : 0.f;
-    wt[3] = (vy1 && vx1) ? ly * lx * m : 0.f;
-  }
-}
 
 // ---- LDS budget per instantiation --------------------------------------------------------------
-template <typename T, typename OutT, int NBF, int MODE> struct DcnLds {
+template <typename T, typename OutT, int NBF> struct DcnLds {
   static constexpr bool BLDS = sizeof(T) == 2;     // 16-bit paths stage the weights in LDS
   static constexpr int NB = NBF * 16;
   static constexpr int PXS = sizeof(T) == 2 ? 40 : 36;  // elements per region pixel (32 + pad: conflict-free rows)
   static constexpr int PXB = PXS * (int)sizeof(T);
-  // FUSED 16-bit stages the 18 offset filters of up to 3 chunks here first (9 x 18 x 104 elements)
-  static constexpr int BCOLS = (MODE == MODE_FUSED && BLDS) ? (NB > 64 ? NB : 64) : (NB > 32 ? NB : 32);
-  static constexpr int BSM = BLDS ? 9 * BCOLS * 32 : 8;
-  static constexpr int NINFO = MODE == MODE_PLAIN ? 1 : DCN_NPAIR;
-  static constexpr int NOFF = MODE == MODE_FUSED ? DCN_TILE * DCN_NOFF : 1;
+  static constexpr int BSM = BLDS ? 9 * (NB > 32 ? NB : 32) * 32 : 8;
   static constexpr int SROW = NB + 16 / (int)sizeof(OutT);  // epilogue staging row (elements)
-  static constexpr int FIXED = BSM * (int)sizeof(T) + NINFO * ((int)sizeof(typename InfoOf<T>::type) + 1) +
-                               NOFF * 4 + 4 * NB * 4 + 256;
   static constexpr int STAGE_BYTES = DCN_TILE * SROW * (int)sizeof(OutT);  // epilogue tile, then GAP rows [waves][NB]
   static constexpr int STAGE_PX = (STAGE_BYTES + DCN_WAVES * NB * 4 + PXB - 1) / PXB;
-  // region staging uses RCAP / DCN_SLOT pieces per thread; the epilogue tile reuses the region
-  static constexpr int RCAP_MIN = STAGE_PX > 768 ? STAGE_PX : 768;
-  static constexpr int RCAP_WANT = (RCAP_MIN + 63) / 64 * 64;
-  static constexpr int RCAP_FIT = (DCN_LDS - FIXED) / PXB < RCAP_WANT ? (DCN_LDS - FIXED) / PXB : RCAP_WANT;
-  static constexpr int RCAP = RCAP_FIT / 64 * 64;    // a multiple of 64 pixels
-  static_assert(RCAP >= DCN_FCAP, "footprint must fit the region buffer");
-  static_assert(MODE == MODE_PLAIN || sizeof(T) == 4 || RCAP * PXB <= 65536, "16-bit corner offsets");
-  static_assert(RCAP * PXB >= STAGE_BYTES + DCN_WAVES * NB * 4, "epilogue tile must fit the region buffer");
-  static_assert(MODE == MODE_PLAIN || RCAP * PXB >= DCN_SE_LDS, "fused SE scratch must fit the region buffer");
+  // footprint buffer (pixels); the epilogue tile reuses it
+  static constexpr int RCAP = ((STAGE_PX > DCN_FCAP ? STAGE_PX : DCN_FCAP) + 63) / 64 * 64;
+  static_assert(RCAP * PXB + BSM * (int)sizeof(T) + 4 * NB * 4 + 256 <= DCN_LDS, "LDS");
 };
-
-// ---- buffer loads ------------------------------------------------------------------------------
-// A raw buffer load returns 0 for a byte offset at or past the descriptor's
-// size, so pieces outside the image (padding ring, channels past Cin, unused
-// staging slots) are staged as zeros with no branch; per-thread byte offsets are
-// computed once per block and only shifted per channel chunk.
-constexpr uint32_t DCN_OOB = KAD_OOB;
-
-template <typename T>
-__device__ __forceinline__ typename DcnFrag<T>::frag buf_ld8(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
-  typedef typename DcnFrag<T>::frag F;
-  if constexpr (sizeof(T) == 4) {
-    F f;
-    f.lo = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-    f.hi = __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(r, voff + 16, 0, 0));
-    return f;
-  } else {
-    return __builtin_bit_cast(F, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-  }
-}
 
 // Chunk staging: up to CAP region pixels x 32 channels, 8-channel pieces,
 // prefetched in registers; piece u of thread t is pixel t / 4 + DCN_SLOT u,
@@ -485,218 +233,15 @@ __device__ __forceinline__ void plain_conv(floatx4 (&acc)[DCN_WM][NBP], __amdgpu
   }
 }
 
-// ---- conv_offset of one tile, 16-bit input ------------------------------------------------------------
-// Up to 3 channel chunks per round trip: the footprint [fpix][GS] goes to
-// `region` and the 18 offset filters [9 taps][18][GS] to `bsm` (GS = 32 G + 8
-// elements: rows 16 bytes apart in bank space, conflict-free for consecutive
-// pixels / filters), all loads of a group issued at once; then 9 G k-steps of
-// 2 x 2 MFMA with no barrier in between.  oacc[m][b]: offset channel 16 b + row.
-template <typename T, int REGION_BYTES, int BSM_BYTES>
-__device__ __forceinline__ void offset_conv16(floatx4 (&oacc)[DCN_WM][2], __amdgpu_buffer_rsrc_t rx,
-                                              __amdgpu_buffer_rsrc_t rw, int nchunk, int cin8, int h, int w,
-                                              int x_cs, int stride, int fy0, int fx0, const DcnGeom& g, T* region,
-                                              T* bsm) {
-  typedef DcnFrag<T> Ops;
-  typedef typename Ops::frag frag;
-  constexpr int NTF = 12, NTW = 8;           // footprint / filter pieces per thread per round
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = lane & 15, grp = lane >> 4;
-  const int fpix = g.fh * g.fw;
-  int apix[DCN_WM];
-#pragma unroll
-  for (int m = 0; m < DCN_WM; ++m) {
-    int pl = wave * (16 * DCN_WM) + m * 16 + row;
-    if (pl >= g.th * g.tw) pl = 0;
-    const int py = (int)(((float)pl + 0.5f) * g.inv_tw), px = pl - py * g.tw;
-    apix[m] = (py * stride) * g.fw + px * stride;
-  }
-  for (int c0 = 0; c0 < nchunk;) {
-    int G = nchunk - c0 < 3 ? nchunk - c0 : 3;
-    while (G > 1 && (fpix * (32 * G + 8) * (int)sizeof(T) > REGION_BYTES ||
-                     9 * DCN_NOFF * (32 * G + 8) * (int)sizeof(T) > BSM_BYTES))
-      --G;
-    const int GS = 32 * G + 8, P4 = 4 * G;
-    const float inv_p4 = 1.f / (float)P4;
-    const int np = fpix * P4, nw = 9 * DCN_NOFF * P4;
-    // one descriptor per pass (a buffer descriptor must be wave-uniform)
-    for (int fb = 0, wb = 0; fb < np || wb < nw; fb += NTF * DCN_THREADS, wb += NTW * DCN_THREADS) {
-      frag vf[NTF], vw[NTW];
-      // pieces past np / nw are skipped by block-uniform branches (no address work, no load)
-#pragma unroll
-      for (int t = 0; t < NTF; ++t) {  // footprint piece: pixel q, 8 channels r of the group
-        vf[t] = zero8<T>();
-        if (fb + t * DCN_THREADS >= np) continue;
-        const int e = fb + tid + t * DCN_THREADS;
-        uint32_t o = DCN_OOB;
-        if (e < np) {
-          const int q = (int)(((float)e + 0.5f) * inv_p4), r = e - q * P4;
-          const int qy = (int)(((float)q + 0.5f) * g.inv_fw), qx = q - qy * g.fw;
-          const int gy = fy0 + qy, gx = fx0 + qx, ch = c0 * 32 + r * 8;
-          if (gy >= 0 && gy < h && gx >= 0 && gx < w && ch < cin8)
-            o = (uint32_t)(((gy * w + gx) * x_cs + ch) * (int)sizeof(T));
-        }
-        vf[t] = buf_ld8<T>(rx, o);
-      }
-#pragma unroll
-      for (int t = 0; t < NTW; ++t) {  // filter piece: tap k, filter col, 8 channels r
-        vw[t] = zero8<T>();
-        if (wb + t * DCN_THREADS >= nw) continue;
-        const int f = wb + tid + t * DCN_THREADS;
-        uint32_t o = DCN_OOB;
-        if (f < nw) {
-          const int kc = (int)(((float)f + 0.5f) * inv_p4), r = f - kc * P4;
-          const int k = kc / DCN_NOFF, col = kc - k * DCN_NOFF;
-          o = (uint32_t)((((col * nchunk + c0 + (r >> 2)) * 9 + k) * 32 + (r & 3) * 8) * (int)sizeof(T));
-        }
-        vw[t] = buf_ld8<T>(rw, o);
-      }
-#pragma unroll
-      for (int t = 0; t < NTF; ++t) {
-        const int e = fb + tid + t * DCN_THREADS;
-        if (e < np) {
-          const int q = (int)(((float)e + 0.5f) * inv_p4), r = e - q * P4;
-          st8<T>(region + q * GS + r * 8, vf[t]);
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < NTW; ++t) {
-        const int f = wb + tid + t * DCN_THREADS;
-        if (f < nw) {
-          const int kc = (int)(((float)f + 0.5f) * inv_p4), r = f - kc * P4;
-          st8<T>(bsm + kc * GS + r * 8, vw[t]);
-        }
-      }
-    }
-    __syncthreads();
-    for (int gi = 0; gi < G; ++gi) {
-      const int cofs = gi * 32 + grp * 8;
-#pragma unroll
-      for (int k = 0; k < 9; ++k) {  // unrolled: the scheduler runs LDS reads ahead of the MFMAs
-        const frag b0 = ld8<T>(bsm + (k * DCN_NOFF + row) * GS + cofs);
-        frag b1 = zero8<T>();
-        if (row < DCN_NOFF - 16) b1 = ld8<T>(bsm + (k * DCN_NOFF + 16 + row) * GS + cofs);
-        const int toff = (k / 3) * g.fw + k % 3;
-#pragma unroll
-        for (int m = 0; m < DCN_WM; ++m) {
-          const frag af = ld8<T>(region + (apix[m] + toff) * GS + cofs);
-          oacc[m][0] = Ops::mma(af, b0, oacc[m][0]);
-          oacc[m][1] = Ops::mma(af, b1, oacc[m][1]);
-        }
-      }
-    }
-    __syncthreads();  // footprint / filters consumed before the next group (or the caller) reuses them
-    c0 += G;
-  }
-}
-
-// ---- fused squeeze-excitation of one image ------------------------------------------------------
-// Cross-block exchange without fences.  A device-scope release fence writes
-// back the whole L2 of the XCD (8 XCDs, each with its own L2), which costs
-// microseconds per block; atomic read-modify-writes, by contrast, are
-// performed at the memory-side coherence point for every XCD.  So every step
-// of the exchange is a relaxed device-scope RMW whose returned value the
-// thread waits for (the RMW has then been performed):
-//  - each block stores its GAP partials with atomic exchanges and waits;
-//  - after a barrier, thread 0 increments the image's arrival counter;
-//  - the block that completes the count resets it (exchange with 0) and reads
-//    every partial of the image with device-scope atomic loads (coherent across
-//    XCDs: they do not return a stale line of the reader's L2).
-// se_tail then forms g = se_inv_count * column sums of the [tiles][Cout]
-// partials in a fixed order (thread (slice s, channel c) takes tiles s,
-// s + nsl, ...; the slices are then added in order), so the result does not
-// depend on which block came last; then att = sigmoid(W2 relu(W1 g + b1) + b2)
-// with 4 lanes per output and a shuffle reduction.  lds: Cout + hid + THREADS floats.
-// (dev_load / rmw_store: kad_common.h)
-
-template <int THREADS>
-__device__ __forceinline__ void se_tail(const float* __restrict__ partial, const float* __restrict__ w1,
-                                        const float* __restrict__ b1, const float* __restrict__ w2,
-                                        const float* __restrict__ b2, float* __restrict__ att, float inv_count, int C,
-                                        int hid, int n, int tiles, float* lds) {
-  constexpr int PB = 16;   // loads in flight per thread per batch
-  constexpr int LPO = 4;   // lanes per MLP output (shuffle-reduced)
-  constexpr int OPP = THREADS / LPO;  // outputs per pass
-  const int tid = threadIdx.x;
-  float* g = lds;          // [C]
-  float* hb = g + C;       // [hid]
-  float* red = hb + hid;   // [nsl][C]
-  const float* pn = partial + (int64_t)n * tiles * C;
-  const int nsl = C < THREADS ? THREADS / C : 1;
-  for (int e = tid; e < nsl * C; e += THREADS) {
-    const int s = e / C, ch = e - s * C;
-    float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int t0 = s; t0 < tiles; t0 += PB * nsl) {
-      float v[PB];
-#pragma unroll
-      for (int u = 0; u < PB; ++u) {
-        const int t = t0 + u * nsl;
-        v[u] = t < tiles ? dev_load(pn + (int64_t)t * C + ch) : 0.f;
-      }
-#pragma unroll
-      for (int u = 0; u < PB; ++u) acc[u & 3] += v[u];
-    }
-    red[e] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-  }
-  __syncthreads();
-  for (int ch = tid; ch < C; ch += THREADS) {
-    float v = 0.f;
-    for (int s = 0; s < nsl; ++s) v += red[s * C + ch];
-    g[ch] = v * inv_count;
-  }
-  __syncthreads();
-  const int part = tid & (LPO - 1);
-  // out[o] = act(sum_k w[o][k] in[k] + b[o]): LPO lanes per output, each taking k = part, part + LPO, ...
-  auto layer = [&](const float* __restrict__ w, const float* __restrict__ b, const float* in, int nin, int nout,
-                   bool relu, float* dst) {
-    for (int o0 = 0; o0 < nout; o0 += OPP) {
-      const int o = o0 + tid / LPO;
-      const float* wr = w + (int64_t)(o < nout ? o : 0) * nin;
-      float acc = 0.f;
-      for (int k0 = part; k0 < nin; k0 += PB * LPO) {
-        float wv[PB];
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-          const int k = k0 + u * LPO;
-          wv[u] = (o < nout && k < nin) ? wr[k] : 0.f;
-        }
-#pragma unroll
-        for (int u = 0; u < PB; ++u) {
-          const int k = k0 + u * LPO;
-          acc += wv[u] * in[k < nin ? k : 0];
-        }
-      }
-      acc += __shfl_xor(acc, 1);
-      acc += __shfl_xor(acc, 2);
-      if (o < nout && part == 0) {
-        const float v = acc + (b ? b[o] : 0.f);
-        dst[o] = relu ? fmaxf(v, 0.f) : sigmoidf_(v);
-      }
-    }
-  };
-  layer(w1, b1, g, C, hid, true, hb);
-  __syncthreads();
-  layer(w2, b2, hb, hid, C, false, att + (int64_t)n * C);
-}
-
 // ---- kernel ------------------------------------------------------------------------------------
-// The block's work: tile-order index bx (XCD-aware, see below) and column block by of ny, of the
-// problem (a, g).  dcn_fwd_kernel runs one problem per launch, dcn_group_kernel several.
-template <typename T, typename OutT, int NBF, int MODE>
-__device__ __forceinline__ void dcn_block(const kad_dcn_args& a, const DcnGeom& g, const int bx, const int by,
-                                          const int ny) {
-  typedef DcnFrag<T> Ops;
-  typedef typename Ops::frag frag;
-  typedef typename InfoOf<T>::type Info;
-  typedef DcnLds<T, OutT, NBF, MODE> L;
-  constexpr int NB = L::NB, PXS = L::PXS, PXB = L::PXB, RCAP = L::RCAP;
-  constexpr bool BLDS = L::BLDS;
-  __shared__ __align__(16) T region[RCAP * PXS];     // input region / footprint; epilogue tile at the end
+template <typename T, typename OutT, int NBF>
+__global__ __launch_bounds__(DCN_THREADS, 1) void plain_kernel(kad_dcn_args a, DcnGeom g) {
+  typedef DcnLds<T, OutT, NBF> L;
+  constexpr int NB = L::NB, PXS = L::PXS, RCAP = L::RCAP;
+  __shared__ __align__(16) T region[RCAP * PXS];     // footprint; epilogue tile at the end
   __shared__ __align__(16) T bsm[L::BSM];            // chunk weights [9][cols][32] (16-bit paths)
-  __shared__ Info s_info[L::NINFO];                  // [9][128] corner offsets + weights
-  __shared__ unsigned char s_slow[L::NINFO];         // [9][128] 1 = sample outside the capped region
-  __shared__ float s_off[L::NOFF];                   // FUSED: [128][18] offsets of the tile
   __shared__ float s_par[4][NB];                     // bias, post_mul, post_add, post_scale
-  __shared__ int s_box[4];       // ymin, ymax, xmin, xmax (clamped corners of live samples)
-  __shared__ int s_reg[5];       // region y0, x0, rows, cols, capped flag
+  const int bx = blockIdx.x, by = blockIdx.y;
 
   // XCD-aware tile order over (image, tile) flattened: block b runs on XCD b % 8, which takes a
   // contiguous run of it (8 images: one image per XCD), so neighbouring tiles share their halos
@@ -718,7 +263,6 @@ __device__ __forceinline__ void dcn_block(const kad_dcn_args& a, const DcnGeom& 
   const __amdgpu_buffer_rsrc_t rwp = make_rsrc(wp, (uint32_t)(g.cout_pad * g.nchunk * 9 * 32 * (int)sizeof(T)));
   const int fy0 = ty0 * a.stride - a.pad, fx0 = tx0 * a.stride - a.pad;
 
-  // ---- 0. independent loads ------------------------------------------------------------------------
   float par[4] = {0.f, 1.f, 0.f, 1.f};
   if (tid < NB) {
     const int co = co0 + tid;
@@ -729,353 +273,16 @@ __device__ __forceinline__ void dcn_block(const kad_dcn_args& a, const DcnGeom& 
       if (a.post_scale) par[3] = a.post_scale[co];
     }
   }
-  // this thread's prologue pixel (taps tid / 128 + KSTEP u)
-  const int ppl = tid & (DCN_TILE - 1);
-  const int ppy = (int)(((float)ppl + 0.5f) * g.inv_tw), ppx = ppl - ppy * g.tw;
-  const int poy = ty0 + ppy, pox = tx0 + ppx;
-  const bool plive = ppl < npx && poy < g.ho && pox < g.wo;
-  const int64_t pp = (int64_t)poy * g.wo + pox;
-  float pre_dy[DCN_PPT], pre_dx[DCN_PPT], pre_m[DCN_PPT];
-  if constexpr (MODE != MODE_PLAIN) {
-#pragma unroll
-    for (int u = 0; u < DCN_PPT; ++u) {
-      const int k = tid / DCN_TILE + DCN_KSTEP * u;
-      pre_dy[u] = pre_dx[u] = 0.f;
-      pre_m[u] = 1.f;
-      if (k < 9 && plive) {
-        if constexpr (MODE == MODE_EXT) {
-          pre_dy[u] = a.offset[n * a.off_sn + pp * a.off_sp + (2 * k) * a.off_sc];
-          pre_dx[u] = a.offset[n * a.off_sn + pp * a.off_sp + (2 * k + 1) * a.off_sc];
-        }
-        if (a.mask) pre_m[u] = a.mask[n * a.mask_sn + pp * a.mask_sp + k * a.mask_sc];
-      }
-    }
-  }
-  if (tid == 0) {
-    s_box[0] = 0x7fffffff;
-    s_box[1] = -1;
-    s_box[2] = 0x7fffffff;
-    s_box[3] = -1;
-  }
-
   floatx4 acc[DCN_WM][NBF];
 #pragma unroll
   for (int m = 0; m < DCN_WM; ++m)
 #pragma unroll
     for (int b = 0; b < NBF; ++b) acc[m][b] = floatx4{0.f, 0.f, 0.f, 0.f};
 
-  if constexpr (MODE == MODE_PLAIN) {
-    // ---- 1. plain 3x3 convolution -----------------------------------------------------------------
-    plain_conv<T, NBF, PXS>(acc, rx, rwp, wp, co0, g.cout_pad, g.nchunk, cin8, a.h, a.w, a.x_cs, a.stride, fy0, fx0,
-                            g, region, bsm);
-  } else {
-    if constexpr (MODE == MODE_FUSED) {
-      // ---- 1. offsets = conv_offset(x) over the tile ----------------------------------------------------
-      floatx4 oacc[DCN_WM][2];
-#pragma unroll
-      for (int m = 0; m < DCN_WM; ++m) oacc[m][0] = oacc[m][1] = floatx4{0.f, 0.f, 0.f, 0.f};
-      const __amdgpu_buffer_rsrc_t rwo = make_rsrc(a.off_wpack, (uint32_t)(32 * g.nchunk * 9 * 32 * (int)sizeof(T)));
-      if constexpr (BLDS)
-        offset_conv16<T, RCAP * PXB, L::BSM * (int)sizeof(T)>(oacc, rx, rwo, g.nchunk, cin8, a.h, a.w, a.x_cs,
-                                                               a.stride, fy0, fx0, g, region, bsm);
-      else
-        plain_conv<T, 2, PXS>(oacc, rx, rwo, (const T*)a.off_wpack, 0, 32, g.nchunk, cin8, a.h, a.w, a.x_cs,
-                              a.stride, fy0, fx0, g, region, bsm);
-#pragma unroll
-      for (int b = 0; b < 2; ++b) {
-        const int ch = b * 16 + row;
-        if (ch < DCN_NOFF) {
-          const float ob = a.off_bias ? a.off_bias[ch] : 0.f;
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              s_off[(wave * (16 * DCN_WM) + m * 16 + grp * 4 + i) * DCN_NOFF + ch] = oacc[m][b][i] + ob;
-        }
-      }
-      __syncthreads();  // offsets visible; footprint buffers free
-    }
-    // ---- 2. samples: clamped corners, weights, bounding box (registers) --------------------------------
-    int bymin = 0x7fffffff, bymax = -1, bxmin = 0x7fffffff, bxmax = -1;
-    int smp_yx[DCN_PPT], smp_st[DCN_PPT];
-    float smp_w[DCN_PPT][4];
-#pragma unroll
-    for (int u = 0; u < DCN_PPT; ++u) {
-      const int k = tid / DCN_TILE + DCN_KSTEP * u;
-      float* w = smp_w[u];
-      w[0] = w[1] = w[2] = w[3] = 0.f;
-      int cy0 = 0, cx0 = 0, sy = 0, sx = 0;
-      if (k < 9 && plive) {
-        const int ky = k / 3, kx = k - (k / 3) * 3;
-        float dy = pre_dy[u], dx = pre_dx[u];
-        if constexpr (MODE == MODE_FUSED) {
-          dy = s_off[ppl * DCN_NOFF + 2 * k];
-          dx = s_off[ppl * DCN_NOFF + 2 * k + 1];
-        }
-        const float py = (float)(poy * a.stride - a.pad + ky) + dy;
-        const float px = (float)(pox * a.stride - a.pad + kx) + dx;
-        sample_geom(py, px, pre_m[u], a.h, a.w, cy0, cx0, sy, sx, w);
-      }
-      const bool live = w[0] != 0.f || w[1] != 0.f || w[2] != 0.f || w[3] != 0.f;
-      if (live) {
-        bymin = min(bymin, cy0);
-        bymax = max(bymax, cy0 + sy);
-        bxmin = min(bxmin, cx0);
-        bxmax = max(bxmax, cx0 + sx);
-      }
-      smp_yx[u] = (cy0 << 15) | cx0;
-      smp_st[u] = (sy << 1) | sx;
-    }
-    // wave-level then block-level bounding box (integer min / max: order-independent)
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      bymin = min(bymin, __shfl_xor(bymin, o));
-      bymax = max(bymax, __shfl_xor(bymax, o));
-      bxmin = min(bxmin, __shfl_xor(bxmin, o));
-      bxmax = max(bxmax, __shfl_xor(bxmax, o));
-    }
-    __syncthreads();  // s_box initialised
-    if (lane == 0) {
-      atomicMin(&s_box[0], bymin);
-      atomicMax(&s_box[1], bymax);
-      atomicMin(&s_box[2], bxmin);
-      atomicMax(&s_box[3], bxmax);
-    }
-    __syncthreads();
-    if (tid == 0) {
-      int ry0 = s_box[0], ry1 = s_box[1], rx0 = s_box[2], rx1 = s_box[3];
-      int capped = 0;
-      if (ry1 < ry0 || rx1 < rx0) {  // no live sample at all
-        ry0 = ry1 = rx0 = rx1 = 0;
-      } else if ((ry1 - ry0 + 1) * (rx1 - rx0 + 1) > RCAP) {
-        // keep the tile's own footprint plus the widest halo m that fits
-        const int fy0c = max(fy0, 0), fy1 = min(fy0 + g.fh - 1, a.h - 1);
-        const int fx0c = max(fx0, 0), fx1 = min(fx0 + g.fw - 1, a.w - 1);
-        int m = 0;
-        while (m < 4096) {
-          const int y0n = max(ry0, fy0c - m - 1), y1n = min(ry1, fy1 + m + 1);
-          const int x0n = max(rx0, fx0c - m - 1), x1n = min(rx1, fx1 + m + 1);
-          if ((y1n - y0n + 1) * (x1n - x0n + 1) > RCAP) break;
-          ++m;
-        }
-        const int y0n = max(ry0, fy0c - m), y1n = min(ry1, fy1 + m);
-        const int x0n = max(rx0, fx0c - m), x1n = min(rx1, fx1 + m);
-        if ((y1n - y0n + 1) * (x1n - x0n + 1) <= RCAP && y1n >= y0n && x1n >= x0n) {
-          ry0 = y0n;
-          ry1 = y1n;
-          rx0 = x0n;
-          rx1 = x1n;
-        } else {  // degenerate (very wide tile footprint): a 1 x 1 region, everything global
-          ry1 = ry0;
-          rx1 = rx0;
-        }
-        capped = 1;
-      }
-      s_reg[0] = ry0;
-      s_reg[1] = rx0;
-      s_reg[2] = ry1 - ry0 + 1;
-      s_reg[3] = rx1 - rx0 + 1;
-      s_reg[4] = capped;
-    }
-    __syncthreads();
-    const int ry0 = s_reg[0], rx0 = s_reg[1], rh = s_reg[2], rw = s_reg[3];
-    const bool block_may_slow = s_reg[4] != 0;
-    const int rpix = rh * rw;
-    const float inv_rw = 1.f / (float)rw;
-    const int gq8 = (tid & 3) * 8;
+  plain_conv<T, NBF, PXS>(acc, rx, rwp, wp, co0, g.cout_pad, g.nchunk, cin8, a.h, a.w, a.x_cs, a.stride, fy0, fx0, g,
+                          region, bsm);
 
-    // ---- 3. chunk 0 in flight while the sample records are written ------------------------------------
-    RegionTile<T, RCAP> rt;
-    WeightTile<T, BLDS ? NB : 1> wt;
-    rt.setup(ry0, rx0, rw, rpix, inv_rw, a.h, a.w, a.x_cs, tid);
-    rt.load(rx, 0, gq8 < cin8);
-    if constexpr (BLDS) {
-      wt.setup(co0, g.cout_pad, g.nchunk, tid);
-      wt.load(rwp, 0);
-    }
-#pragma unroll
-    for (int u = 0; u < DCN_PPT; ++u) {
-      const int k = tid / DCN_TILE + DCN_KSTEP * u;
-      if (k >= 9) break;
-      const int q = k * DCN_TILE + ppl;
-      float* w = smp_w[u];
-      const int cy0 = smp_yx[u] >> 15, cx0 = smp_yx[u] & 0x7fff;
-      const int sy = smp_st[u] >> 1, sx = smp_st[u] & 1;
-      const int ly = cy0 - ry0, lx = cx0 - rx0;
-      const bool dead = w[0] == 0.f && w[1] == 0.f && w[2] == 0.f && w[3] == 0.f;
-      unsigned o[4] = {0u, 0u, 0u, 0u};
-      unsigned char slow = 0;
-      if (!dead && ly >= 0 && ly + sy < rh && lx >= 0 && lx + sx < rw) {
-        const unsigned b0 = (unsigned)((ly * rw + lx) * PXB);
-        const unsigned bxs = (unsigned)(sx * PXB), bys = (unsigned)(sy * rw * PXB);
-        o[0] = b0;
-        o[1] = b0 + bxs;
-        o[2] = b0 + bys;
-        o[3] = b0 + bys + bxs;
-      } else {
-        slow = dead ? 0 : 1;            // the fast path skips it; the slow pass adds it
-        w[0] = w[1] = w[2] = w[3] = 0.f;
-      }
-      s_info[q] = make_info<T>(o, w);
-      s_slow[q] = slow;
-    }
-    rt.store(region, PXS, tid);
-    if constexpr (BLDS) wt.store(bsm, tid);
-
-    const int ibase = wave * (16 * DCN_WM) + row;      // this lane's pixel slot within a tap row of s_info
-    const T* wrow[NBF];                                // this lane's weight row (output channel) per fragment
-#pragma unroll
-    for (int b = 0; b < NBF; ++b) {
-      const int co = co0 + b * 16 + row;
-      wrow[b] = wp + (int64_t)(co < g.cout_pad ? co : 0) * g.nchunk * 9 * 32 + grp * 8;
-    }
-    for (int c = 0; c < g.nchunk; ++c) {
-      __syncthreads();
-      if (c + 1 < g.nchunk) {  // in flight during this chunk's taps
-        rt.load(rx, c + 1, (c + 1) * 32 + gq8 < cin8);
-        if constexpr (BLDS) wt.load(rwp, c + 1);
-      }
-      // lanes whose channel group lies past Cin read staged zeros: no masking needed
-      frag bn[NBF];
-      if constexpr (!BLDS) {
-#pragma unroll
-        for (int b = 0; b < NBF; ++b) bn[b] = ld8<T>(wrow[b] + (c * 9) * 32);
-      }
-      if constexpr (BLDS) {
-        // Software-pipelined taps (fully unrolled, so the buffers rotate without
-        // moves): the LDS reads of tap k + 1 (weights, corners) and the sample
-        // records of tap k + 2 are in flight while tap k blends and multiplies.
-        const char* rb = (const char*)region + grp * 8 * (int)sizeof(T);
-        Info inf[3][DCN_WM];
-        frag bq[2][NBF], cq[2][DCN_WM][4];
-        auto rd_info = [&](int k, Info (&d)[DCN_WM]) {
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m) d[m] = s_info[k * DCN_TILE + m * 16 + ibase];
-        };
-        auto rd_tap = [&](int k, const Info (&in)[DCN_WM], frag (&bd)[NBF], frag (&cd)[DCN_WM][4]) {
-#pragma unroll
-          for (int b = 0; b < NBF; ++b) bd[b] = b_read<T, NB>(bsm, k, b * 16 + row, grp);
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) cd[m][j] = ld8<T>((const T*)(rb + corner(in[m], j)));
-        };
-        rd_info(0, inf[0]);
-        rd_info(1, inf[1]);
-        rd_tap(0, inf[0], bq[0], cq[0]);
-#pragma unroll
-        for (int k = 0; k < 9; ++k) {
-          const int cur = k & 1, nxt = cur ^ 1;
-          if (k + 2 < 9) rd_info(k + 2, inf[(k + 2) % 3]);
-          if (k + 1 < 9) rd_tap(k + 1, inf[(k + 1) % 3], bq[nxt], cq[nxt]);
-          frag af[DCN_WM];
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m)
-            af[m] = Ops::blend(cq[cur][m][0], cq[cur][m][1], cq[cur][m][2], cq[cur][m][3], inf[k % 3][m]);
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m)
-#pragma unroll
-            for (int b = 0; b < NBF; ++b) acc[m][b] = Ops::mma(af[m], bq[cur][b], acc[m][b]);
-        }
-      } else {
-      Info ic[DCN_WM], inx[DCN_WM];
-#pragma unroll
-      for (int m = 0; m < DCN_WM; ++m) inx[m] = s_info[m * 16 + ibase];
-#pragma unroll 1
-      for (int k = 0; k < 9; ++k) {
-#pragma unroll
-        for (int m = 0; m < DCN_WM; ++m) ic[m] = inx[m];
-        if (k < 8) {
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m) inx[m] = s_info[(k + 1) * DCN_TILE + m * 16 + ibase];
-        }
-        frag bf[NBF];
-        {
-#pragma unroll
-          for (int b = 0; b < NBF; ++b) bf[b] = bn[b];
-          if (k < 8) {
-#pragma unroll
-            for (int b = 0; b < NBF; ++b) bn[b] = ld8<T>(wrow[b] + (c * 9 + k + 1) * 32);
-          }
-        }
-        frag af[DCN_WM];
-#pragma unroll
-        for (int m = 0; m < DCN_WM; ++m) {
-          const char* rb = (const char*)region + grp * 8 * (int)sizeof(T);
-          const frag v0 = ld8<T>((const T*)(rb + corner(ic[m], 0)));
-          const frag v1 = ld8<T>((const T*)(rb + corner(ic[m], 1)));
-          const frag v2 = ld8<T>((const T*)(rb + corner(ic[m], 2)));
-          const frag v3 = ld8<T>((const T*)(rb + corner(ic[m], 3)));
-          af[m] = Ops::blend(v0, v1, v2, v3, ic[m]);
-        }
-#pragma unroll
-        for (int m = 0; m < DCN_WM; ++m)
-#pragma unroll
-          for (int b = 0; b < NBF; ++b) acc[m][b] = Ops::mma(af[m], bf[b], acc[m][b]);
-      }
-      }
-      if (c + 1 < g.nchunk) {
-        __syncthreads();  // every wave is done with this chunk's region and weights
-        rt.store(region, PXS, tid);
-        if constexpr (BLDS) wt.store(bsm, tid);
-      }
-    }
-
-    // ---- 3c. samples outside a capped region: straight from global memory (rare) ----------------------
-    if (block_may_slow) {
-      // The wave stays converged up to every MFMA (MFMA needs all 64 lanes):
-      // lanes past Cin contribute zero fragments instead of branching away.
-      for (int c = 0; c < g.nchunk; ++c) {
-        const int ch = c * 32 + grp * 8;
-        const bool ch_ok = ch < cin8;
-#pragma unroll 1
-        for (int k = 0; k < 9; ++k) {
-          frag af[DCN_WM];
-          bool any = false;
-#pragma unroll
-          for (int m = 0; m < DCN_WM; ++m) {
-            const int q = k * DCN_TILE + m * 16 + ibase;
-            af[m] = zero8<T>();
-            if (ch_ok && s_slow[q]) {
-              // recompute the sample's geometry (rare path)
-              const int pl = m * 16 + ibase;
-              const int oyl = (int)(((float)pl + 0.5f) * g.inv_tw);
-              const int oy = ty0 + oyl, ox = tx0 + pl - oyl * g.tw;
-              const int64_t p = (int64_t)oy * g.wo + ox;
-              float dy, dx;
-              if constexpr (MODE == MODE_FUSED) {
-                dy = s_off[pl * DCN_NOFF + 2 * k];
-                dx = s_off[pl * DCN_NOFF + 2 * k + 1];
-              } else {
-                dy = a.offset[n * a.off_sn + p * a.off_sp + (2 * k) * a.off_sc];
-                dx = a.offset[n * a.off_sn + p * a.off_sp + (2 * k + 1) * a.off_sc];
-              }
-              const float mk = a.mask ? a.mask[n * a.mask_sn + p * a.mask_sp + k * a.mask_sc] : 1.f;
-              int cy0, cx0, sy, sx;
-              float w[4];
-              sample_geom((float)(oy * a.stride - a.pad + k / 3) + dy, (float)(ox * a.stride - a.pad + k % 3) + dx,
-                          mk, a.h, a.w, cy0, cx0, sy, sx, w);
-              const unsigned o0[4] = {0u, 0u, 0u, 0u};
-              const Info in = make_info<T>(o0, w);
-              const T* g0 = xb + ((int64_t)cy0 * a.w + cx0) * a.x_cs + ch;
-              af[m] = Ops::blend(ld8<T>(g0), ld8<T>(g0 + sx * a.x_cs), ld8<T>(g0 + (int64_t)sy * a.w * a.x_cs),
-                                 ld8<T>(g0 + ((int64_t)sy * a.w + sx) * a.x_cs), in);
-              any = true;
-            }
-          }
-          if (__builtin_amdgcn_ballot_w64(any) == 0) continue;
-#pragma unroll
-          for (int b = 0; b < NBF; ++b) {
-            const frag bw = ld8<T>(wrow[b] + (c * 9 + k) * 32);
-#pragma unroll
-            for (int m = 0; m < DCN_WM; ++m) acc[m][b] = Ops::mma(af[m], bw, acc[m][b]);
-          }
-        }
-      }
-    }
-  }
-
-  // ---- 4. epilogue: values -> LDS tile -> row-contiguous stores; GAP partials ------------------------
+  // ---- epilogue: values -> LDS tile -> row-contiguous stores; GAP partials ------------------------
   constexpr int SROW = L::SROW;
   OutT* ost = (OutT*)region;
   float(*gap_red)[NB] = (float(*)[NB])((char*)region + L::STAGE_BYTES);
@@ -1188,78 +395,16 @@ __device__ __forceinline__ void dcn_block(const kad_dcn_args& a, const DcnGeom& 
       float v = 0.f;
 #pragma unroll
       for (int i = 0; i < DCN_WAVES; ++i) v += gap_red[i][tid];
-      float* dst = a.gap_partial + ((int64_t)n * g.tiles + tile) * a.cout + co;
-      if (MODE != MODE_PLAIN && a.se_att)
-        rmw_store(dst, v);  // read by another block of this launch (fused SE)
-      else
-        *dst = v;
-    }
-  }
-
-  // ---- 5. fused squeeze-excitation: the image's last block runs the MLP -------------------------------
-  // (exchange protocol at se_tail)
-  if constexpr (MODE != MODE_PLAIN) {
-    if (a.se_att && a.gap_partial) {
-      __shared__ int s_last;
-      // This block's partial exchanges are performed (each thread waited for its exchange's
-      // return) and the epilogue's LDS tile is free.  The barrier waits for LDS traffic only,
-      // not for the acknowledgements of the output stores, which no one here reads.
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (tid == 0) {
-        const unsigned total = (unsigned)g.tiles * ny;
-        const unsigned prev = __hip_atomic_fetch_add(a.se_count + n, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int last = prev + 1u == total;
-        if (last) {
-          const unsigned z = __hip_atomic_exchange(a.se_count + n, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          asm volatile("" ::"v"(z));
-        }
-        s_last = last;
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      if (s_last) {
-        se_tail<DCN_THREADS>(a.gap_partial, a.se_w1, a.se_b1, a.se_w2, a.se_b2, a.se_att, a.se_inv_count, a.cout, a.se_hid, n,
-                g.tiles, (float*)region);
-      }
+      a.gap_partial[((int64_t)n * g.tiles + tile) * a.cout + co] = v;
     }
   }
 }
 
-template <typename T, typename OutT, int NBF, int MODE>
-__global__ __launch_bounds__(DCN_THREADS, 1) void dcn_fwd_kernel(kad_dcn_args a, DcnGeom g) {
-  dcn_block<T, OutT, NBF, MODE>(a, g, blockIdx.x, blockIdx.y, gridDim.y);
-}
-
-// Several independent problems of one instantiation (same dtype, mode and column-fragment count)
-// in one grid: problem p owns blocks [start[p], start[p + 1]) (its grid_x x ny blocks, start a
-// multiple of 8 so a block's XCD, id % 8, is its tile order's).  The three branches of a KAD-Conv
-// layer run their DSCs this way, as one launch instead of three concurrent streams.
-struct DcnGroup {
-  kad_dcn_args a[KAD_DCN_GROUP_MAX];
-  DcnGeom g[KAD_DCN_GROUP_MAX];
-  int start[KAD_DCN_GROUP_MAX + 1];
-  int ny[KAD_DCN_GROUP_MAX];
-  int count;
-};
-
-template <typename T, typename OutT, int NBF, int MODE>
-__global__ __launch_bounds__(DCN_THREADS, 1) void dcn_group_kernel(DcnGroup grp) {
-  const int id = blockIdx.x;
-  int p = 0;
-#pragma unroll
-  for (int i = 1; i < KAD_DCN_GROUP_MAX; ++i)
-    if (i < grp.count && id >= grp.start[i]) p = i;
-  if (id >= grp.start[p + 1]) return;
-  const int local = id - grp.start[p];
-  const int gx = grp.g[p].grid_x;
-  // p is uniform over the block: the problem's fields are scalar loads from kernel-argument memory
-  dcn_block<T, OutT, NBF, MODE>(grp.a[p], grp.g[p], local % gx, local / gx, grp.ny[p]);
-}
-
-// ---- 16-bit DCN / DSC with two blocks per CU ------------------------------------------------------
-// The 16-bit FUSED and EXT paths at stride 1 with up to 64 output channels and many tiles (KAD-CNet's
-// small DSCs; the dispatch rule and its measurements are at d2_ok).  On gfx950 LDS delivers ~128 B/clk per CU and L1 hits ~64 B/clk; the
-// tap loop of the 8-wave kernel above is bound by LDS reads, most of them weight fragments that
-// every wave re-reads for its 16 pixels.  Here:
+// ---- narrow 16-bit DCN / DSC, two or three blocks per CU ------------------------------------------
+// The 16-bit FUSED and EXT paths at stride 1 with up to 16 output channels (KAD-CNet's first-level
+// DSCs).  Against the gathering kernel (us, fp16 DSC alone, this / gathering): Cout 10 at
+// [16, 100, 100] 25 / 36, [8, 100, 100] 15 / 23, [8, 50, 50] 10.6 / 11.3; but Cout 24 at [16, 100, 100]
+// 42 / 37 and Cout 64 85 / 61 (four column fragments): those run there.  Here:
 //  * 4 waves x 32 pixels (two 16-pixel A fragments per wave): half the weight-fragment reads per
 //    pixel, and they come from global memory (L1 / L2 hits: a column block's packed weights are
 //    at most 9 x 64 x 64 x 2 bytes), so LDS carries only the corner reads;
@@ -1286,7 +431,6 @@ constexpr int D2_RCAP = 1024;                  // region pixels per half-chunk b
 constexpr int D2_RBUF = D2_RCAP * 32;          // bytes per region buffer
 // shared area (conv_offset staging, offsets, region buffers, epilogue, SE): NRB * D2_RBUF bytes
 constexpr int D2_RINST = D2_RCAP * 2 / 64 / D2_WAVES;  // direct loads per wave per half-chunk
-constexpr int D2_NBF_MAX = 4;
 constexpr unsigned D2_SLOW = 0x80000000u;      // record flag: sample outside the region (read from memory)
 static_assert(DCN_TILE == D2_TILE && D2_THREADS / D2_TILE == 2, "sample geometry");
 
@@ -1375,10 +519,11 @@ __device__ __forceinline__ void d2_offset_conv(floatx4 (&oacc)[2][2], __amdgpu_b
 // NRB: region buffers.  One suffices when Cin <= 16 (a single half-chunk, nothing to prefetch): the
 // block then needs ~46 KB of LDS instead of ~78 KB, three blocks per CU instead of two (the host
 // checks that the conv_offset staging and the SE scratch fit the smaller shared area).
-template <typename T, int NBF, int MODE, int NRB>
+template <typename T, int MODE, int NRB>
 __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom& g, const int bx, const int by,
                                            const int ny) {
-  static_assert(sizeof(T) == 2 && NBF <= D2_NBF_MAX && MODE != MODE_PLAIN, "16-bit DCN / DSC only");
+  static_assert(sizeof(T) == 2 && MODE != MODE_PLAIN, "16-bit DCN / DSC only");
+  constexpr int NBF = 1;  // 16-channel column fragments
   static_assert(NRB == 1 || NRB == 2, "one or two region buffers");
   typedef DcnFrag<T> Ops;
   typedef typename Ops::frag frag;
@@ -1912,17 +1057,17 @@ __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom&
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (s_last)
-      se_tail<D2_THREADS>(a.gap_partial, a.se_w1, a.se_b1, a.se_w2, a.se_b2, a.se_att, a.se_inv_count, a.cout,
+      se_tail<D2_THREADS, SU / 4>(a.gap_partial, a.se_w1, a.se_b1, a.se_w2, a.se_b2, a.se_att, a.se_inv_count, a.cout,
                           a.se_hid, n, g.tiles, (float*)s_u);
   }
 }
 
-template <typename T, int NBF, int MODE, int NRB>
+template <typename T, int MODE, int NRB>
 __global__ __launch_bounds__(D2_THREADS, 2) void dsc2_kernel(kad_dcn_args a, DcnGeom g) {
-  dsc2_block<T, NBF, MODE, NRB>(a, g, blockIdx.x, blockIdx.y, gridDim.y);
+  dsc2_block<T, MODE, NRB>(a, g, blockIdx.x, blockIdx.y, gridDim.y);
 }
 
-template <typename T, int NBF, int NRB>
+template <typename T, int NRB>
 __global__ __launch_bounds__(D2_THREADS, 2) void dsc2_group_kernel(DcnGroup grp) {
   const int id = blockIdx.x;
   int p = 0;
@@ -1932,7 +1077,7 @@ __global__ __launch_bounds__(D2_THREADS, 2) void dsc2_group_kernel(DcnGroup grp)
   if (id >= grp.start[p + 1]) return;
   const int local = id - grp.start[p];
   const int gx = grp.g[p].grid_x;
-  dsc2_block<T, NBF, MODE_FUSED, NRB>(grp.a[p], grp.g[p], local % gx, local / gx, grp.ny[p]);
+  dsc2_block<T, MODE_FUSED, NRB>(grp.a[p], grp.g[p], local % gx, local / gx, grp.ny[p]);
 }
 
 // ---- weight packing ------------------------------------------------------------------------------
@@ -1951,42 +1096,25 @@ __global__ void dcn_pack_kernel(const float* w, T* out, int cin, int cout, int n
   }
 }
 
-static DcnGeom make_geom(const kad_dcn_args& a, int ho, int wo) {
-  DcnGeom g;
-  g.ho = ho;
-  g.wo = wo;
-  pick_tile(ho, wo, &g.th, &g.tw);
-  g.tiles_x = ceil_div(wo, g.tw);
-  g.tiles = ceil_div(ho, g.th) * g.tiles_x;
-  g.grid_x = round_up(a.n * g.tiles, 8);  // flattened (image, tile), padded to whole XCD rounds
-  g.nchunk = ceil_div(a.cin, 32);
-  g.cout_pad = round_up(a.cout, 16);
-  g.fh = (g.th - 1) * a.stride + 3;
-  g.fw = (g.tw - 1) * a.stride + 3;
-  g.inv_tw = 1.f / (float)g.tw;
-  g.inv_fw = 1.f / (float)g.fw;
-  return g;
-}
-
-template <typename T, typename OutT, int NBF, int MODE>
-static int launch_dcn(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
+template <typename T, typename OutT, int NBF>
+static int launch_plain(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
   dim3 grid(g.grid_x, ceil_div(a.cout, NBF * 16), 1);
-  hipLaunchKernelGGL((dcn_fwd_kernel<T, OutT, NBF, MODE>), grid, dim3(DCN_THREADS), 0, st, a, g);
-  return check_launch(MODE == MODE_PLAIN ? "kad_conv3x3_fwd" : MODE == MODE_FUSED ? "kad_dsc_fwd" : "kad_dcn_fwd");
+  hipLaunchKernelGGL((plain_kernel<T, OutT, NBF>), grid, dim3(DCN_THREADS), 0, st, a, g);
+  return check_launch("kad_conv3x3_fwd");
 }
 
-template <typename T, typename OutT, int MODE>
-static int dispatch_dcn(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
+template <typename T, typename OutT>
+static int dispatch_plain(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
   const int nbf = ceil_div(a.cout, 16);
   switch (nbf < 8 ? nbf : 8) {
-    case 1: return launch_dcn<T, OutT, 1, MODE>(a, st, g);
-    case 2: return launch_dcn<T, OutT, 2, MODE>(a, st, g);
-    case 3: return launch_dcn<T, OutT, 3, MODE>(a, st, g);
-    case 4: return launch_dcn<T, OutT, 4, MODE>(a, st, g);
-    case 5: return launch_dcn<T, OutT, 5, MODE>(a, st, g);
-    case 6: return launch_dcn<T, OutT, 6, MODE>(a, st, g);
-    case 7: return launch_dcn<T, OutT, 7, MODE>(a, st, g);
-    default: return launch_dcn<T, OutT, 8, MODE>(a, st, g);
+    case 1: return launch_plain<T, OutT, 1>(a, st, g);
+    case 2: return launch_plain<T, OutT, 2>(a, st, g);
+    case 3: return launch_plain<T, OutT, 3>(a, st, g);
+    case 4: return launch_plain<T, OutT, 4>(a, st, g);
+    case 5: return launch_plain<T, OutT, 5>(a, st, g);
+    case 6: return launch_plain<T, OutT, 6>(a, st, g);
+    case 7: return launch_plain<T, OutT, 7>(a, st, g);
+    default: return launch_plain<T, OutT, 8>(a, st, g);
   }
 }
 
@@ -2032,19 +1160,9 @@ static int validate_dcn(const kad_dcn_args* a, int mode, DcnGeom* g_out) {
 using namespace kad;
 
 namespace kad {
-// The two-blocks-per-CU kernel: 16-bit, stride 1, at most D2_COUT_MAX output channels (one column
-// block), and enough blocks (>= D2_MIN_BLOCKS over all problems of a launch) for two to share a
-// CU.  Measured per launch on KAD-CNet-S (bs16, 800^2, fp16): 1680 blocks of Cout <= 16: 90 ->
-// 59 us; 432 blocks: 33 -> 22 us; but 128 blocks of Cout 32: 19.8 -> 21.7 us (one 4-wave block
-// per CU), and the KAD-Conv(256) branches (Cout 86 at 100^2 / 50^2 / 25^2: 640 / 160 / 40
-// blocks) 87 / 32 / 31 -> 89 / 44 / 44 us.  Everything else runs on dcn_fwd_kernel.
-constexpr int D2_COUT_MAX = 16 * D2_NBF_MAX;
-constexpr int64_t D2_MIN_BLOCKS = 384;
-static bool d2_shape_ok(const kad_dcn_args& a) {
-  return (a.dtype == KAD_F16 || a.dtype == KAD_BF16) && a.stride == 1 && a.cout <= D2_COUT_MAX;
-}
-static bool d2_ok(const kad_dcn_args& a, const DcnGeom& g) {
-  return d2_shape_ok(a) && (int64_t)a.n * g.tiles >= D2_MIN_BLOCKS;
+// The narrow kernel: 16-bit, stride 1, at most 16 output channels.
+static bool d2_ok(const kad_dcn_args& a) {
+  return (a.dtype == KAD_F16 || a.dtype == KAD_BF16) && a.stride == 1 && a.cout <= 16;
 }
 // One region buffer (NRB = 1): a single 16-channel half-chunk, and the conv_offset staging of one
 // 32-channel chunk (footprint and filters, 5 slots per row) and the SE scratch within D2_RBUF.
@@ -2054,49 +1172,29 @@ static bool d2_single(const kad_dcn_args& a, const DcnGeom& g) {
          (a.cout + a.se_hid + D2_THREADS) * 4 <= D2_RBUF;
 }
 
-template <typename T, int NBF, int MODE>
+template <typename T, int MODE>
 static int launch_d2(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
   if (d2_single(a, g))
-    hipLaunchKernelGGL((dsc2_kernel<T, NBF, MODE, 1>), dim3(g.grid_x, 1, 1), dim3(D2_THREADS), 0, st, a, g);
+    hipLaunchKernelGGL((dsc2_kernel<T, MODE, 1>), dim3(g.grid_x), dim3(D2_THREADS), 0, st, a, g);
   else
-    hipLaunchKernelGGL((dsc2_kernel<T, NBF, MODE, 2>), dim3(g.grid_x, 1, 1), dim3(D2_THREADS), 0, st, a, g);
+    hipLaunchKernelGGL((dsc2_kernel<T, MODE, 2>), dim3(g.grid_x), dim3(D2_THREADS), 0, st, a, g);
   return check_launch(MODE == MODE_FUSED ? "kad_dsc_fwd" : "kad_dcn_fwd");
 }
 
-template <typename T, int MODE>
-static int dispatch_d2(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
-  switch (ceil_div(a.cout, 16)) {
-    case 1: return launch_d2<T, 1, MODE>(a, st, g);
-    case 2: return launch_d2<T, 2, MODE>(a, st, g);
-    case 3: return launch_d2<T, 3, MODE>(a, st, g);
-    default: return launch_d2<T, 4, MODE>(a, st, g);
-  }
-}
-
 template <int MODE>
-static int dispatch_d2_dtype(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
-  return a.dtype == KAD_F16 ? dispatch_d2<half_t, MODE>(a, st, g) : dispatch_d2<bf16_t, MODE>(a, st, g);
+static int dispatch_d2(const kad_dcn_args& a, hipStream_t st, const DcnGeom& g) {
+  return a.dtype == KAD_F16 ? launch_d2<half_t, MODE>(a, st, g) : launch_d2<bf16_t, MODE>(a, st, g);
 }
 
-template <typename T, int NBF>
+template <typename T>
 static int launch_group_d2(const DcnGroup& grp, hipStream_t st) {
   bool single = true;
   for (int p = 0; p < grp.count; ++p) single = single && d2_single(grp.a[p], grp.g[p]);
   if (single)
-    hipLaunchKernelGGL((dsc2_group_kernel<T, NBF, 1>), dim3(grp.start[grp.count]), dim3(D2_THREADS), 0, st, grp);
+    hipLaunchKernelGGL((dsc2_group_kernel<T, 1>), dim3(grp.start[grp.count]), dim3(D2_THREADS), 0, st, grp);
   else
-    hipLaunchKernelGGL((dsc2_group_kernel<T, NBF, 2>), dim3(grp.start[grp.count]), dim3(D2_THREADS), 0, st, grp);
+    hipLaunchKernelGGL((dsc2_group_kernel<T, 2>), dim3(grp.start[grp.count]), dim3(D2_THREADS), 0, st, grp);
   return check_launch("kad_dsc_fwd_group");
-}
-
-template <typename T>
-static int dispatch_group_d2(const DcnGroup& grp, int nbf, hipStream_t st) {
-  switch (nbf) {
-    case 1: return launch_group_d2<T, 1>(grp, st);
-    case 2: return launch_group_d2<T, 2>(grp, st);
-    case 3: return launch_group_d2<T, 3>(grp, st);
-    default: return launch_group_d2<T, 4>(grp, st);
-  }
 }
 }  // namespace kad
 
@@ -2134,9 +1232,9 @@ extern "C" int kad_conv3x3_fwd(const kad_dcn_args* a, void* stream) {
   if (rc) return fail(rc, "kad_conv3x3_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
   switch (a->dtype) {
-    case KAD_F32: return dispatch_dcn<float, float, MODE_PLAIN>(*a, st, g);
-    case KAD_F16: return dispatch_dcn<half_t, float, MODE_PLAIN>(*a, st, g);
-    case KAD_BF16: return dispatch_dcn<bf16_t, float, MODE_PLAIN>(*a, st, g);
+    case KAD_F32: return dispatch_plain<float, float>(*a, st, g);
+    case KAD_F16: return dispatch_plain<half_t, float>(*a, st, g);
+    case KAD_BF16: return dispatch_plain<bf16_t, float>(*a, st, g);
     default: return fail(KAD_EINVAL, "kad_conv3x3_fwd: unknown dtype %d", a->dtype);
   }
 }
@@ -2150,9 +1248,9 @@ extern "C" int kad_conv_fwd(const kad_dcn_args* a, void* stream) {
   rc = convolution_igemm(*a, g.ho, g.wo, st);  // 16-bit, NHWC output: implicit-GEMM kernel
   if (rc != 1) return rc;
   switch (a->dtype) {
-    case KAD_F32: return dispatch_dcn<float, float, MODE_PLAIN>(*a, st, g);
-    case KAD_F16: return dispatch_dcn<half_t, half_t, MODE_PLAIN>(*a, st, g);
-    case KAD_BF16: return dispatch_dcn<bf16_t, bf16_t, MODE_PLAIN>(*a, st, g);
+    case KAD_F32: return dispatch_plain<float, float>(*a, st, g);
+    case KAD_F16: return dispatch_plain<half_t, half_t>(*a, st, g);
+    case KAD_BF16: return dispatch_plain<bf16_t, bf16_t>(*a, st, g);
     default: return fail(KAD_EINVAL, "kad_conv_fwd: unknown dtype %d", a->dtype);
   }
 }
@@ -2162,11 +1260,11 @@ extern "C" int kad_dcn_fwd(const kad_dcn_args* a, void* stream) {
   int rc = validate_dcn(a, MODE_EXT, &g);
   if (rc) return fail(rc, "kad_dcn_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
-  if (d2_ok(*a, g)) return dispatch_d2_dtype<MODE_EXT>(*a, st, g);
+  if (d2_ok(*a)) return dispatch_d2<MODE_EXT>(*a, st, g);
   switch (a->dtype) {
-    case KAD_F32: return dispatch_dcn<float, float, MODE_EXT>(*a, st, g);
-    case KAD_F16: return dispatch_dcn<half_t, half_t, MODE_EXT>(*a, st, g);
-    case KAD_BF16: return dispatch_dcn<bf16_t, bf16_t, MODE_EXT>(*a, st, g);
+    case KAD_F32: return dcn_gather<float>(*a, g, MODE_EXT, st);
+    case KAD_F16: return dcn_gather<half_t>(*a, g, MODE_EXT, st);
+    case KAD_BF16: return dcn_gather<bf16_t>(*a, g, MODE_EXT, st);
     default: return fail(KAD_EINVAL, "kad_dcn_fwd: unknown dtype %d", a->dtype);
   }
 }
@@ -2176,37 +1274,14 @@ extern "C" int kad_dsc_fwd(const kad_dcn_args* a, void* stream) {
   int rc = validate_dcn(a, MODE_FUSED, &g);
   if (rc) return fail(rc, "kad_dsc_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
-  if (d2_ok(*a, g)) return dispatch_d2_dtype<MODE_FUSED>(*a, st, g);
+  if (d2_ok(*a)) return dispatch_d2<MODE_FUSED>(*a, st, g);
   switch (a->dtype) {
-    case KAD_F32: return dispatch_dcn<float, float, MODE_FUSED>(*a, st, g);
-    case KAD_F16: return dispatch_dcn<half_t, half_t, MODE_FUSED>(*a, st, g);
-    case KAD_BF16: return dispatch_dcn<bf16_t, bf16_t, MODE_FUSED>(*a, st, g);
+    case KAD_F32: return dcn_gather<float>(*a, g, MODE_FUSED, st);
+    case KAD_F16: return dcn_gather<half_t>(*a, g, MODE_FUSED, st);
+    case KAD_BF16: return dcn_gather<bf16_t>(*a, g, MODE_FUSED, st);
     default: return fail(KAD_EINVAL, "kad_dsc_fwd: unknown dtype %d", a->dtype);
   }
 }
-
-namespace kad {
-template <typename T, typename OutT, int NBF>
-static int launch_group(const DcnGroup& grp, hipStream_t st) {
-  hipLaunchKernelGGL((dcn_group_kernel<T, OutT, NBF, MODE_FUSED>), dim3(grp.start[grp.count]), dim3(DCN_THREADS), 0,
-                     st, grp);
-  return check_launch("kad_dsc_fwd_group");
-}
-
-template <typename T, typename OutT>
-static int dispatch_group(const DcnGroup& grp, int nbf, hipStream_t st) {
-  switch (nbf) {
-    case 1: return launch_group<T, OutT, 1>(grp, st);
-    case 2: return launch_group<T, OutT, 2>(grp, st);
-    case 3: return launch_group<T, OutT, 3>(grp, st);
-    case 4: return launch_group<T, OutT, 4>(grp, st);
-    case 5: return launch_group<T, OutT, 5>(grp, st);
-    case 6: return launch_group<T, OutT, 6>(grp, st);
-    case 7: return launch_group<T, OutT, 7>(grp, st);
-    default: return launch_group<T, OutT, 8>(grp, st);
-  }
-}
-}  // namespace kad
 
 extern "C" int kad_dsc_fwd_group(const kad_dcn_args* a, int count, void* stream) {
   KAD_CHECK_ARG(a && count >= 1 && count <= KAD_DCN_GROUP_MAX, "kad_dsc_fwd_group: count %d outside [1, %d]", count,
@@ -2231,16 +1306,13 @@ extern "C" int kad_dsc_fwd_group(const kad_dcn_args* a, int count, void* stream)
   grp.start[count] = (int)blocks;
   for (int p = count + 1; p <= KAD_DCN_GROUP_MAX; ++p) grp.start[p] = (int)blocks;
   hipStream_t st = (hipStream_t)stream;
-  bool all_d2 = blocks >= D2_MIN_BLOCKS;
-  for (int p = 0; p < count; ++p) all_d2 = all_d2 && d2_shape_ok(a[p]);
-  if (all_d2) {
-    if (a[0].dtype == KAD_F16) return dispatch_group_d2<half_t>(grp, nbf, st);
-    return dispatch_group_d2<bf16_t>(grp, nbf, st);
-  }
+  bool all_d2 = true;
+  for (int p = 0; p < count; ++p) all_d2 = all_d2 && d2_ok(a[p]);
+  if (all_d2) return a[0].dtype == KAD_F16 ? launch_group_d2<half_t>(grp, st) : launch_group_d2<bf16_t>(grp, st);
   switch (a[0].dtype) {
-    case KAD_F32: return dispatch_group<float, float>(grp, nbf, st);
-    case KAD_F16: return dispatch_group<half_t, half_t>(grp, nbf, st);
-    case KAD_BF16: return dispatch_group<bf16_t, bf16_t>(grp, nbf, st);
+    case KAD_F32: return dcn_gather_group<float>(grp, nbf, st);
+    case KAD_F16: return dcn_gather_group<half_t>(grp, nbf, st);
+    case KAD_BF16: return dcn_gather_group<bf16_t>(grp, nbf, st);
     default: return fail(KAD_EINVAL, "kad_dsc_fwd_group: unknown dtype %d", a[0].dtype);
   }
 }

@@ -29,10 +29,8 @@ import torch
 from . import _ext
 
 
-DCN_BLOCK_COLS = 128  # output channels per block of the DCN kernels (8 MFMA column fragments)
-SPLIT_MIN_TILES = 128  # tiles per launch from which a separate offset conv pays (half the CUs)
 GROUPED = True         # KADConvPlan: branch stages as grouped launches on one stream for small layers
-GROUP_MAX_WORK = 2048  # ... whose full-resolution DSC has less work: N x tiles x column fragments
+GROUP_MAX_WORK = 1600  # ... whose full-resolution DSC has less work: N x tiles x column fragments
 
 
 def _f32(t):
@@ -140,20 +138,9 @@ class DSCPlan:
             st.append(('lcsa_mask' + tag, lambda: _ext.lcsa_mask(arow, colm, self.lcsa, emat, ebias, mask, n,
                                                                  self.cin, h, w, ks, work)))
         b = self.bias if bias is None else bias
-        if self.cout > DCN_BLOCK_COLS and se is None and n * _ext.dcn_tiles(h, w) >= SPLIT_MIN_TILES:
-            # several 128-channel column blocks per tile: conv_offset once per tile (a plain 3x3 conv
-            # into an fp32 [N, h, w, 18] map), then the deformable conv reading those offsets, instead
-            # of every column block of the fused kernel recomputing the same offsets.  With few tiles
-            # the separate offset launch occupies few CUs and costs more than it saves (measured:
-            # [8,256,50,50] 166 -> 158 us split; [8,512,25,25], 40 tiles, 153 -> 156 us).
-            off = torch.empty(n, h, w, 18, dtype=torch.float32, device=dev)
-            st.append(('conv_offset' + tag, lambda: _ext.conv3x3_fwd(y, self.cin, owp, 18, off, bias=self.off_b)))
-            st.append(('dsc' + tag, lambda: _ext.dcn_fwd(
-                y, self.cin, off, (P * 18, 18, 1), mask, (P * 9, 9, 1), wp, self.cout, out, bias=b,
-                post_mul=post_mul, post_add=post_add, post_scale=post_scale, relu=relu, out_layout=out_layout,
-                gap_partial=gap)))
-            return st
-        # conv_offset + deformable conv in one kernel: the offsets stay on chip
+        # conv_offset + deformable conv in one kernel: the offsets stay on chip.  Above 128 output channels
+        # every column block forms them again, which still beats a conv_offset launch of its own (fp16 DSC,
+        # one launch / two): [8,256,50,50] 112 / 119 us, [8,256,100,100] 280 / 293, [8,512,25,25] 120 / 135.
         st.append(('dsc' + tag, lambda: _ext.dsc_fwd(
             y, self.cin, owp, self.off_b, mask, (P * 9, 9, 1), wp, self.cout, out, bias=b, post_mul=post_mul,
             post_add=post_add, post_scale=post_scale, relu=relu, out_layout=out_layout, gap_partial=gap, se=se)))
@@ -234,9 +221,10 @@ class KADConvPlan:
         latency, and under HIP-graph replay the three side-stream chains of a small layer
         were measured to run one after another (KAD-CNet-S: 9.62 -> 9.14 ms per batch with
         every KADC4 grouped).  A heavy layer keeps the side streams: the coarse branches'
-        DSCs and merges then fill the last, partly empty round of the full-resolution DSC
-        (KADConv(256) at [8, 256, 100, 100], 640 tiles x 6 fragments: 210 us with streams,
-        227 us grouped)."""
+        DSCs and merges then fill the full-resolution DSC's last, partly empty round.
+        fp16 layers, grouped / streams (us; work): KADConv(256) [4, 75, 75] 122 / 132 (1.1k),
+        KADConv(192) [8, 80, 80] 103 / 102 (1.7k), KADConv(128) [8, 100, 100] 129 / 121 (1.9k),
+        KADConv(256) [16, 50, 50] 166 / 167 (1.9k), KADConv(256) [8, 100, 100] 180 / 167 (3.8k)."""
         frags = min((self.branches[0].c + 15) // 16, 8)
         work = x.shape[0] * _ext.dcn_tiles(x.shape[2], x.shape[3]) * frags
         return self.groupable and work < GROUP_MAX_WORK

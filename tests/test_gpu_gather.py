@@ -1,0 +1,97 @@
+"""Edges of the gathering deformable convolution and of its fused squeeze-excitation tail,
+against the CPU oracle (tolerances of tests/_util.check_close: fp32 1e-4 of the output scale,
+16-bit 1e-2).  Output channels around the 16 / 32 / 96 / 128-channel borders of the dispatch and of
+the column blocks, input channels that leave a 64-byte step partly empty, odd and even counts of
+steps, tiles with one row, stride 2 (footprints larger than the prefetch registers hold, one LDS
+buffer instead of two), samples far outside the tile and the image."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from oracle import kadconv_oracle as O
+from tests._util import check_close, nhwc_padded, quant
+
+pytestmark = pytest.mark.gpu
+
+DT = {'f32': torch.float32, 'f16': torch.float16, 'bf16': torch.bfloat16}
+
+
+def _case(N, C, Co, H, W, stride, off_std, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    Ho, Wo = (H - 1) // stride + 1, (W - 1) // stride + 1
+    x = torch.randn(N, C, H, W, generator=g)
+    ow = torch.randn(18, C, 3, 3, generator=g) * (off_std / (9 * C) ** 0.5)
+    ob = torch.randn(18, generator=g) * 0.3
+    w = (torch.rand(Co, C, 3, 3, generator=g) * 2 - 1) / (9 * C) ** 0.5
+    b = torch.randn(Co, generator=g) * 0.1
+    mask = torch.rand(N, 9, Ho, Wo, generator=g)
+    off = F.conv2d(quant(x, dtype), quant(ow, dtype), ob.double(), stride=stride, padding=1)
+    ref = O.deform_conv2d(quant(x, dtype), off, quant(w, dtype), b.double(), stride=stride, padding=1,
+                          mask=mask.double())
+    return x, ow, ob, w, b, mask, off, ref
+
+
+@pytest.mark.parametrize('dt', ['f16', 'bf16', 'f32'])
+@pytest.mark.parametrize('mode', ['dsc', 'dcn'])
+@pytest.mark.parametrize('shape,stride,off_std', [
+    ((2, 8, 17, 11, 13), 1, 2.0), ((1, 24, 32, 16, 9), 1, 2.0), ((2, 31, 33, 12, 25), 1, 3.0),
+    ((1, 65, 96, 20, 21), 1, 2.0), ((1, 33, 97, 9, 30), 1, 2.0), ((1, 130, 129, 14, 11), 1, 2.0),
+    ((1, 48, 48, 1, 200), 1, 1.0), ((1, 40, 40, 50, 2), 1, 40.0), ((2, 16, 20, 25, 41), 2, 2.0),
+    ((1, 20, 36, 5, 257), 2, 2.0), ((1, 72, 64, 67, 9), 2, 30.0)])
+def test_gather_edges(dt, mode, shape, stride, off_std):
+    from kadconv import _ext
+    dtype = DT[dt]
+    N, C, Co, H, W = shape
+    x, ow, ob, w, b, mask, off, ref = _case(*shape, stride, off_std, dtype, seed=sum(shape))
+    Ho, Wo = ref.shape[2:]
+    print(f'gather {dt} {mode} {shape} stride={stride} off_std={off_std}', flush=True)
+    xq = nhwc_padded(x.to(dtype).cuda())
+    md = mask.permute(0, 2, 3, 1).contiguous().cuda()
+    wp = _ext.dcn_pack_weights(w.to(dtype).cuda(), dtype)
+    for layout in (_ext.KAD_NCHW, _ext.KAD_NHWC):
+        cs = (Co + 7) // 8 * 8
+        out = torch.empty(N, Co, Ho, Wo, dtype=dtype, device='cuda') if layout == _ext.KAD_NCHW else \
+            torch.full((N, Ho, Wo, cs), 7.0, dtype=dtype, device='cuda')
+        if mode == 'dsc':
+            owp = _ext.dcn_pack_weights(ow.to(dtype).cuda(), dtype)
+            _ext.dsc_fwd(xq, C, owp, ob.cuda(), md, (Ho * Wo * 9, 9, 1), wp, Co, out, stride=stride, bias=b.cuda(),
+                         out_layout=layout)
+        else:
+            _ext.dcn_fwd(xq, C, off.float().permute(0, 2, 3, 1).contiguous().cuda(), (Ho * Wo * 18, 18, 1), md,
+                         (Ho * Wo * 9, 9, 1), wp, Co, out, stride=stride, bias=b.cuda(), out_layout=layout)
+        torch.cuda.synchronize()
+        if layout == _ext.KAD_NHWC:
+            assert (out[..., Co:] == 7.0).all()  # channels past Cout belong to the caller
+            out = out[..., :Co].permute(0, 3, 1, 2)
+        check_close(out, ref, dtype, f'{dt} {mode} {shape} layout {layout}')
+
+
+@pytest.mark.parametrize('c,hid', [(10, 32), (16, 16), (40, 40), (86, 86), (90, 91), (128, 128), (85, 7)])
+def test_se_tail_sizes(c, hid):
+    """Fused squeeze-excitation with weights that fit the LDS beside the partials and ones that do not
+    (c = 90 x 91 and 128 x 128 take the general tail): att against the oracle's MLP on the mean of the
+    kernel's own output, to fp32 rounding of sums of at most 128 terms (1e-5 on values in (0, 1))."""
+    from kadconv import _ext
+    dtype = torch.float16
+    N, H, W = 3, 33, 47
+    x, ow, ob, w, b, mask, _, _ = _case(N, c, c, H, W, 1, 2.0, dtype, seed=c + hid)
+    g = torch.Generator().manual_seed(c * hid)
+    w1, b1 = torch.randn(hid, c, generator=g) / c ** 0.5, torch.randn(hid, generator=g) * 0.1
+    w2, b2 = torch.randn(c, hid, generator=g) / hid ** 0.5, torch.randn(c, generator=g) * 0.1
+    print(f'se tail c={c} hid={hid}', flush=True)
+    att = torch.empty(N, c, device='cuda')
+    count = torch.zeros(N, dtype=torch.int32, device='cuda')
+    gap = torch.empty(N, _ext.dcn_tiles(H, W), c, device='cuda')
+    out = torch.empty(N, c, H, W, dtype=dtype, device='cuda')
+    for _ in range(2):  # the counters are left zero
+        att.fill_(-1)
+        _ext.dsc_fwd(nhwc_padded(x.to(dtype).cuda()), c, _ext.dcn_pack_weights(ow.to(dtype).cuda(), dtype), ob.cuda(),
+                     mask.permute(0, 2, 3, 1).contiguous().cuda(), (H * W * 9, 9, 1),
+                     _ext.dcn_pack_weights(w.to(dtype).cuda(), dtype), c, out, bias=b.cuda(),
+                     out_layout=_ext.KAD_NCHW, gap_partial=gap,
+                     se=(w1.cuda(), b1.cuda(), w2.cuda(), b2.cuda(), att, count))
+        torch.cuda.synchronize()
+        m = out.double().cpu().mean((2, 3))
+        ref = torch.sigmoid(F.linear(torch.relu(F.linear(m, w1.double(), b1.double())), w2.double(), b2.double()))
+        assert (att.double().cpu() - ref).abs().max().item() <= 1e-5
+    assert (count == 0).all()
