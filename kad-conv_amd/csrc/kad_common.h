@@ -135,6 +135,10 @@ inline void allow_lds(F* kernel, size_t bytes) {
 // handles (the caller then runs its general path), else 0 or a KAD_E* code.
 int convolution_igemm(const kad_dcn_args& a, int ho, int wo, hipStream_t st);
 
+// The fp32 paths of kad_gemm1x1_fwd and of kad_conv_fwd / kad_conv3x3_fwd (kad_f32.hip), likewise.
+int gemm_f32(const kad_gemm_args& a, hipStream_t st);
+int conv_f32(const kad_dcn_args& a, int ho, int wo, hipStream_t st);
+
 inline int dtype_size(int dtype) {
   return dtype == KAD_F32 ? 4 : 2;
 }

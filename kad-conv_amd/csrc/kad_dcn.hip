@@ -1232,7 +1232,7 @@ extern "C" int kad_conv3x3_fwd(const kad_dcn_args* a, void* stream) {
   if (rc) return fail(rc, "kad_conv3x3_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
   switch (a->dtype) {
-    case KAD_F32: return dispatch_plain<float, float>(*a, st, g);
+    case KAD_F32: rc = conv_f32(*a, g.ho, g.wo, st); return rc != 1 ? rc : dispatch_plain<float, float>(*a, st, g);
     case KAD_F16: return dispatch_plain<half_t, float>(*a, st, g);
     case KAD_BF16: return dispatch_plain<bf16_t, float>(*a, st, g);
     default: return fail(KAD_EINVAL, "kad_conv3x3_fwd: unknown dtype %d", a->dtype);
@@ -1245,7 +1245,8 @@ extern "C" int kad_conv_fwd(const kad_dcn_args* a, void* stream) {
   if (rc) return fail(rc, "kad_conv_fwd: %s", kad_last_error());
   KAD_CHECK_ARG(a->relu >= KAD_ACT_NONE && a->relu <= KAD_ACT_SILU, "kad_conv_fwd: unknown activation %d", a->relu);
   hipStream_t st = (hipStream_t)stream;
-  rc = convolution_igemm(*a, g.ho, g.wo, st);  // 16-bit, NHWC output: implicit-GEMM kernel
+  rc = a->dtype == KAD_F32 ? conv_f32(*a, g.ho, g.wo, st)            // NHWC output, no post_*
+                           : convolution_igemm(*a, g.ho, g.wo, st);  // NHWC output: implicit-GEMM kernel
   if (rc != 1) return rc;
   switch (a->dtype) {
     case KAD_F32: return dispatch_plain<float, float>(*a, st, g);

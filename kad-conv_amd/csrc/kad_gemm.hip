@@ -757,6 +757,9 @@ static int dispatch_gemm(const kad_gemm_args& a, hipStream_t st, int hp, int wp)
   if constexpr (sizeof(T) == 2) {
     if (nchw_fast_ok(a)) return launch_gemm_nchw<T>(a, st);
     if (nhwc_fast_ok(a)) return launch_gemm_nhwc<T>(a, st);
+  } else {
+    const int rc = gemm_f32(a, st);
+    if (rc != 1) return rc;
   }
   const int ncols = a.out_layout == KAD_NHWC ? round_up(a.cout, 8) : a.cout;
   const int nbf = ceil_div(ncols, 16);
