@@ -510,6 +510,41 @@ int64_t kad_nms_mask_words(int n);
  * torchvision.ops.nms call of non_max_suppression (KAD-CNet/utils/general.py:961). */
 int kad_nms(const float *boxes, unsigned long long *mask, unsigned char *keep, int n, float iou_thr, void *stream);
 
+/* ------------------------------------------------------------------------ */
+/* A fixed list of calls (a small KAD-Conv layer's launches) in one entry     */
+/* ------------------------------------------------------------------------ */
+enum { KAD_CALL_PYRAMID = 0, KAD_CALL_LCSA_PREP = 1, KAD_CALL_LCSA_MASK = 2, KAD_CALL_DSC = 3, KAD_CALL_MERGE = 4,
+       KAD_CALL_SCALE_RESIDUAL = 5 };
+
+/* kad_scale_residual's arguments as a struct */
+typedef struct kad_scale_args {
+  void *out;
+  const float *att;
+  const void *residual;
+  int n, c, h, w, img_c, c_off, layout, dtype;
+} kad_scale_args;
+
+/* args: byte offset in the list's blob of kad_pyramid_args, kad_lcsa_args[count], kad_dcn_args[count],
+ * kad_merge_args or kad_scale_args; arg: kad_lcsa_mask_group's emat_dtype. */
+typedef struct kad_call {
+  int fn, count;
+  int64_t args;
+  int arg;
+} kad_call;
+
+/* The pointer at byte offset `at` of the blob is bases[base] + add. */
+typedef struct kad_reloc {
+  int64_t at, add;
+  int base;
+} kad_reloc;
+
+/* Runs the calls in order on `stream`, with the blob's pointers set from `bases` in a copy of it
+ * (nothing is written to the caller's arrays): what calling the entry points one by one with those
+ * arguments does, each with its own checks.  No reference counterpart (host cost of a small layer).
+ * blob_bytes <= 16384. */
+int kad_run_calls(const void *blob, int64_t blob_bytes, const kad_call *calls, int ncalls, const kad_reloc *relocs,
+                  int nrelocs, void *const *bases, int nbases, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

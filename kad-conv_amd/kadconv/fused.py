@@ -30,6 +30,7 @@ from . import _ext
 
 
 GROUPED = True         # KADConvPlan: branch stages as grouped launches on one stream for small layers
+MAX_LISTS = 16         # KADConvPlan: input geometries whose recorded launches are kept
 GROUP_MAX_WORK = 1600  # ... whose full-resolution DSC has less work: N x tiles x column fragments
 
 
@@ -213,6 +214,7 @@ class KADConvPlan:
             raise NotImplementedError('the fused forward covers n <= 3 branches (the paper uses 3)')
         # grouped: the branches' LCSA and DSC stages run as one launch each (all branches), on the
         # caller's stream; else each branch chain runs on a side stream of its own (see _grouped)
+        self._lists = {}
         self.groupable = GROUPED and all(br.dsc.use_mask for br in self.branches)
 
     def _grouped(self, x):
@@ -271,9 +273,16 @@ class KADConvPlan:
         means, the LCSA masks and the fused DSCs (+ SE) of all branches as one launch each
         (kad_lcsa_prep_group, kad_lcsa_mask_group, kad_dsc_fwd_group), then the merges.
         Returns (stages, out)."""
+        xin, _, out, _, _ = self._io(x, out)
+        st, _, out = self._stages_grouped(x, xin, out)
+        return st, out
+
+    def _stages_grouped(self, x, xin, out):
+        """schedule_grouped's stages on xin and out as _io gives them, their scratch tensors, out."""
         N, C, H, W = x.shape
         dev, dtype = x.device, x.dtype
-        xin, in_layout, out, out_v, out_layout = self._io(x, out)
+        in_layout = out_layout = _ext.KAD_NHWC if _channels_last_view(x) else _ext.KAD_NCHW
+        out_v = out.permute(0, 2, 3, 1) if out_layout == _ext.KAD_NHWC else out
         ntx, nty = _ext.pyramid_tiles(H, W)
         pyr, lcsa, dcn, keep, merges = [], [], {}, [], []
         edt = _emat_dtype(dtype)
@@ -307,7 +316,7 @@ class KADConvPlan:
                               post_mul=br.bn_a, post_add=br.bn_b, post_scale=br.scale, relu=True,
                               out_layout=z_layout, gap_partial=gap, se=se)
             dcn.setdefault(min((br.c + 15) // 16, 8), []).append(a)   # one launch per instantiation
-            keep += [y, rows, cols, arow, colm, mask, gap, z, att]
+            keep += [y, rows, cols, arow, colm, mask, gap, att] + ([] if full else [z])
             merges.append((full, {'z': z, 'c': br.c, 'c_off': br.c_off, 'att': att}))
         st.append(('pyramid', lambda: _ext.pyramid_proj(xin, in_layout, C, pyr)))
         st.append(('lcsa_prep', lambda keep=keep: _ext.lcsa_prep_group(lcsa)))
@@ -326,7 +335,7 @@ class KADConvPlan:
             if up:  # the upsampled branches' windows are contiguous: one band merge
                 lo, hi = up[0]['c_off'], up[-1]['c_off'] + up[-1]['c']
                 st.append(('merge', lambda: _ext.branch_merge(out_v, out_layout, up, residual=xin, channels=(lo, hi))))
-        return st, out
+        return st, keep, out
 
     def schedule(self, x, out=None):
         """(pre, [per-branch stages], post, out): the branch chains (LCSA, DSC,
@@ -421,10 +430,27 @@ class KADConvPlan:
         stream, the branch chains forked onto side streams (concurrent on the GPU;
         HIP-graph capture records the fork/join as graph edges), merge after the join.
         out: see _io (channels-last input only)."""
+        # A small layer's launches cost the host more than the GPU: a geometry's second call records them,
+        # later ones replay them as one native call on one workspace (KADConv(64) [1, 64, 80, 80] fp32,
+        # eager: 161 -> 65 us per call, 62 of them on the GPU).
+        key = (x.shape, x.stride(), x.dtype, x.device, None if out is None else out.stride())
+        lst = self._lists.get(key) if self.groupable else None
+        if lst is not None:
+            xin, _, out, out_v, _ = self._io(x, out)
+            ws = torch.empty(lst.sizes[2], dtype=torch.uint8, device=x.device)
+            lst.run(xin.data_ptr(), out_v.data_ptr(), ws.data_ptr())
+            return out
         if self._grouped(x):
-            st, out = self.schedule_grouped(x, out)
-            for _, fn in st:
-                fn()
+            xin, _, out, out_v, _ = self._io(x, out)
+            st, scratch, out = self._stages_grouped(x, xin, out)
+            run = lambda: [fn() for _, fn in st]  # noqa: E731
+            if key in self._lists:
+                self._lists[key] = _ext.CallList(run, ([xin], [out_v], scratch))
+                return out
+            run()
+            if len(self._lists) >= MAX_LISTS:
+                self._lists.pop(next(iter(self._lists)), None)
+            self._lists[key] = None
             return out
         pre, chains, post, out = self.schedule(x, out)
         for _, fn in pre:
