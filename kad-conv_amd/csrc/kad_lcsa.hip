@@ -230,27 +230,24 @@ template <> struct LmFrag<float> {
   }
 };
 
-constexpr int LM_SC = 96;                              // channels per staged group (3 chunks)
-constexpr int LM_SCS = LM_SC + 4;                       // fp32 row stride of the staged group
-
 // grid (ceil(W/16), ceil(H/16), N).  Wave v computes tile rows 4v..4v+3 (4 MFMA
 // column fragments of 16 pixels each) for all 16 (9 used) mask logits.
-// Per group of up to 96 channels, one round trip brings the block's column
-// means (26 columns: 16 + the 11-tap halo), row means (26 rows) and the
-// strip-conv / BN parameters into LDS; alpha / beta of the 16 columns are
-// formed there once.  Per 32-channel chunk: the lanes' E fragments (11 taps) are
-// requested first, u = relu(alpha a + beta) is written to LDS meanwhile, then
-// 11 x 4 MFMAs.
-// SC: channels per staged group (LM_SC; 32 when every problem has one 32-channel chunk, which cuts
-// the block's LDS from ~71 KB to ~46 KB: three blocks per CU instead of two).
-template <typename ET, int SC = LM_SC>
+// Per 32-channel chunk, one round trip brings the block's column means (26 columns: 16 + the
+// 11-tap halo), row means (26 rows) and the strip-conv / BN parameters into LDS, requested while
+// the previous chunk is worked on; alpha / beta of the 16 columns are formed there, u =
+// relu(alpha a + beta) is written to LDS, then 11 x 4 MFMAs with the lanes' E fragments (11 taps).
+// Bound by the chunk's chain of barriers and, with fp32 E, by the matrix cores.  Chunks share
+// nothing: staging three of them together took one barrier less each, but 71 KB of LDS (97 KB with
+// fp32 E: one block per CU) instead of 46 KB (73 KB), and all of it for a split's single chunk (us,
+// fp16 E / fp32 E, three chunks -> one): C = 128 on [8, 100, 100] 21.1 / 75.9 -> 19.7 / 61.8, C = 512 on
+// [8, 25, 25] 19.4 / 36.6 -> 13.7 / 24.3, C = 12 on [16, 100, 100] 18.0 / 49.9 -> 13.5 / 36.2.
+template <typename ET>
 __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* colm, const float* params,
                                                 const ET* emat, const float* ebias, float* mask, int c, int h, int w,
                                                 int cp, int ksplit, float* part, const int bx, const int by,
                                                 const int bz, const int nz) {
   constexpr int LDU = LmCfg<ET>::ldu;
-  constexpr int SCS = SC + 4;
-  static_assert(SC % 32 == 0 && SC <= LM_SC, "whole 32-channel chunks");
+  constexpr int SC = 32, SCS = SC + 4;
   __shared__ __align__(16) ET us[LM_UR * LM_TW * LDU];
   __shared__ __align__(16) float s_col[LM_UR][SCS];   // column means, columns w0 - 5 .. w0 + 20
   __shared__ __align__(16) float s_a[LM_UR][SCS];     // row means, rows h0 - 5 .. h0 + 20
@@ -281,7 +278,6 @@ __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* 
   constexpr int NW = (LM_UR * SC + LM_THREADS - 1) / LM_THREADS;    // per window
   constexpr int NP = (SC * BAND + LM_THREADS - 1) / LM_THREADS;     // w1
   constexpr int NQ = (3 * SC + LM_THREADS - 1) / LM_THREADS;        // b1 | bn_a | bn_b
-  constexpr int CPG = SC / 32;                                      // chunks per group
   const int nk = cp / 32;
   const int kc0 = sp * nk / ksplit, kc1 = (sp + 1) * nk / ksplit;
   float vc_[NW], va_[NW], vw_[NP], vq_[NQ];
@@ -291,21 +287,21 @@ __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* 
   // c or past the group read 0.
 #define LM_LOAD_GROUP(CS)                                                                                      \
   {                                                                                                            \
-    const int cs_ = (CS), nsc_ = cp - cs_ < SC ? cp - cs_ : SC;                                          \
+    const int cs_ = (CS);                                                                                      \
     _Pragma("unroll") for (int u = 0; u < NW; ++u) {                                                           \
       const int e = tid + u * LM_THREADS, r = e / SC, ch = e - r * SC, gc = cs_ + ch;                    \
       const int gx = w0 - HALF_BAND + r, gy = h0 - HALF_BAND + r;                                              \
-      const bool ok = r < LM_UR && ch < nsc_ && gc < c;                                                        \
+      const bool ok = r < LM_UR && gc < c;                                                                     \
       vc_[u] = (ok && gx >= 0 && gx < w) ? colm_n[(uint32_t)(gx * c + gc)] : 0.f;                              \
       va_[u] = (ok && gy >= 0 && gy < h) ? arow_n[(uint32_t)(gy * c + gc)] : 0.f;                              \
     }                                                                                                          \
     _Pragma("unroll") for (int u = 0; u < NP; ++u) {                                                           \
       const int e = tid + u * LM_THREADS;                                                                      \
-      vw_[u] = (e < nsc_ * BAND && cs_ * BAND + e < c * BAND) ? w1[cs_ * BAND + e] : 0.f;                      \
+      vw_[u] = (e < SC * BAND && cs_ * BAND + e < c * BAND) ? w1[cs_ * BAND + e] : 0.f;                      \
     }                                                                                                          \
     _Pragma("unroll") for (int u = 0; u < NQ; ++u) {                                                           \
       const int e = tid + u * LM_THREADS, which = e / SC, ch = e - which * SC, gc = cs_ + ch;            \
-      vq_[u] = (which < 3 && ch < nsc_ && gc < c) ? (which == 0 ? b1 : which == 1 ? bna : bnb)[gc] : 0.f;      \
+      vq_[u] = (which < 3 && gc < c) ? (which == 0 ? b1 : which == 1 ? bna : bnb)[gc] : 0.f;      \
     }                                                                                                          \
   }
   // this lane's E fragments of chunk KC: logit row l16, taps 0..10, channels 32 KC + grp * 8 .. + 8
@@ -316,14 +312,13 @@ __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* 
   // logit biases, read in the epilogue after many barriers; loaded first, so that their LDS
   // store waits for this load only, not for the group's and the E fragments' loads behind it
   const float ebv = tid < 9 ? ebias[tid] : 0.f;
-  LM_LOAD_GROUP((kc0 / CPG) * SC);
+  LM_LOAD_GROUP(kc0 * SC);
   LM_LOAD_E(kc0);
   if (tid < 16) s_eb[tid] = ebv;
   for (int kc = kc0; kc < kc1; ++kc) {
-    const int g = kc / CPG, c0 = (kc - g * CPG) * 32, cs = g * SC;
-    if (c0 == 0 || kc == kc0) {  // first chunk of a group (or of the split): stage it, request the next one
-      const int nsc = cp - cs < SC ? cp - cs : SC;
-      LM_LDS_BARRIER();  // the previous group's LDS data is consumed
+    const int cs = kc * SC;
+    {  // stage the chunk's means and parameters, request the next chunk's
+      LM_LDS_BARRIER();  // the previous chunk's LDS data is consumed
 #pragma unroll
       for (int u = 0; u < NW; ++u) {
         const int e = tid + u * LM_THREADS, r = e / SC, ch = e - r * SC;
@@ -344,31 +339,31 @@ __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* 
       }
       LM_LDS_BARRIER();
       // strip-conv coefficients of the 16 columns (separable 1x11 conv + folded BN): task
-      // (channel ch, quarter qc of the columns) holds the channel's 11 taps and the 14 column
-      // means its 4 columns need in registers and forms the 4 sliding sums.  The staged column
+      // (channel ch, column pair qc), one per thread, holds the channel's 11 taps and the 12 column
+      // means its 2 columns need in registers and forms the 2 sliding sums.  The staged column
       // means are 0 outside the image, so only S needs the in-image mask.
-      static_assert(LM_TW == 16, "four column quarters");
-      for (int e = tid; e < 4 * SC; e += LM_THREADS) {
-        const int qc = e / SC, ch = e - qc * SC;
-        float wk[BAND], cm[4 + BAND - 1];
+      static_assert(LM_TW / 2 * SC == LM_THREADS, "one task per thread");
+      {
+        const int qc = tid / SC, ch = tid - qc * SC;
+        float wk[BAND], cm[2 + BAND - 1];
 #pragma unroll
         for (int k = 0; k < BAND; ++k) wk[k] = s_w1[ch * BAND + k];
 #pragma unroll
-        for (int j = 0; j < 4 + BAND - 1; ++j) cm[j] = s_col[qc * 4 + j][ch];
-        const bool chok = ch < nsc && cs + ch < c;
+        for (int j = 0; j < 2 + BAND - 1; ++j) cm[j] = s_col[qc * 2 + j][ch];
+        const bool chok = cs + ch < c;
         const float bna = s_bna[ch], bb = s_b1[ch], bnb = s_bnb[ch];
-        // 1 / 0: window column j (image column w0 + 4 qc - 5 + j) inside / outside the image.
+        // 1 / 0: window column j (image column w0 + 2 qc - 5 + j) inside / outside the image.
         // S sums the in-image taps as fma(wk, ind, S): S + wk * 1 and S + wk * 0 round exactly
         // like S + wk and S + 0 (finite weights), with one instruction per tap instead of three.
-        float ind[4 + BAND - 1];
+        float ind[2 + BAND - 1];
 #pragma unroll
-        for (int j = 0; j < 4 + BAND - 1; ++j) {
-          const int xx = w0 + qc * 4 - HALF_BAND + j;
+        for (int j = 0; j < 2 + BAND - 1; ++j) {
+          const int xx = w0 + qc * 2 - HALF_BAND + j;
           ind[j] = (xx >= 0 && xx < w) ? 1.f : 0.f;
         }
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int col = qc * 4 + q, gx = w0 + col;
+        for (int q = 0; q < 2; ++q) {
+          const int col = qc * 2 + q, gx = w0 + col;
           float S0 = 0.f, S1 = 0.f, B0 = 0.f, B1 = 0.f;  // even / odd taps, added last
 #pragma unroll
           for (int k = 0; k < BAND; ++k) {
@@ -386,14 +381,14 @@ __device__ __forceinline__ void lcsa_mask_block(const float* arow, const float* 
           s_beta[col][ch] = ok ? bna * (B + bb) + bnb : 0.f;
         }
       }
-      if ((g + 1) * CPG < kc1) LM_LOAD_GROUP(cs + SC);  // after the coefficients: fewer live registers there
+      if (kc + 1 < kc1) LM_LOAD_GROUP(cs + SC);  // after the coefficients: fewer live registers there
     }
     LM_LDS_BARRIER();  // alpha / beta ready; the previous chunk's MFMAs are done with us
     // u = relu(alpha * a + beta): thread (column, 8-channel group) fixed, rows r0, r0 + 4, ...;
     // its alpha / beta are read once per chunk, one 16-byte LDS store per row
     {
     const int gq = tid & 3, col = (tid >> 2) & (LM_TW - 1), r0 = tid >> 6;
-    const int ch = c0 + gq * 8;
+    const int ch = gq * 8;
     const floatx4 al0 = *(const floatx4*)&s_alpha[col][ch], al1 = *(const floatx4*)&s_alpha[col][ch + 4];
     const floatx4 be0 = *(const floatx4*)&s_beta[col][ch], be1 = *(const floatx4*)&s_beta[col][ch + 4];
     [[maybe_unused]] const half8_t alh =
@@ -464,7 +459,7 @@ __global__ __launch_bounds__(LM_THREADS, 2) void lcsa_mask_kernel(const float* a
                                                                  const float* ebias, float* mask, int c, int h,
                                                                  int w, int cp, int ksplit, float* part) {
   lcsa_mask_block<ET>(arow, colm, params, emat, ebias, mask, c, h, w, cp, ksplit, part, blockIdx.x, blockIdx.y,
-                      blockIdx.z, gridDim.z);
+                          blockIdx.z, gridDim.z);
 }
 
 // Several LCSA problems (the branches of a KAD-Conv layer) in one launch: problem p owns blocks
@@ -475,8 +470,8 @@ struct LcsaGroup {
   int count;
 };
 
-template <typename ET, int SC>
-__global__ __launch_bounds__(LM_THREADS, SC == 32 ? 3 : 2) void lcsa_mask_group_kernel(LcsaGroup grp) {
+template <typename ET>
+__global__ __launch_bounds__(LM_THREADS, sizeof(ET) == 2 ? 3 : 2) void lcsa_mask_group_kernel(LcsaGroup grp) {
   const int id = blockIdx.x;
   int p = 0;
 #pragma unroll
@@ -485,7 +480,7 @@ __global__ __launch_bounds__(LM_THREADS, SC == 32 ? 3 : 2) void lcsa_mask_group_
   const kad_lcsa_args& a = grp.a[p];
   const int local = id - grp.start[p];
   const int tx = ceil_div(a.w, LM_TW), ty = ceil_div(a.h, LM_TH);
-  lcsa_mask_block<ET, SC>(a.arow, a.colm, a.params, (const ET*)a.emat, a.ebias, a.mask, a.c, a.h, a.w,
+  lcsa_mask_block<ET>(a.arow, a.colm, a.params, (const ET*)a.emat, a.ebias, a.mask, a.c, a.h, a.w,
                           round_up(a.c, 32), 1, nullptr, local % tx, (local / tx) % ty, local / (tx * ty), a.n);
 }
 
@@ -526,6 +521,7 @@ __global__ __launch_bounds__(256) void lcsa_mask_reduce_kernel(const float* part
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   float v = 0.f;
+#pragma unroll 8
   for (int s = 0; s < ksplit; ++s) v += part[s * total + i];
   mask[i] = mask_sigmoid(v + ebias[i % 9]);
 }
@@ -715,16 +711,10 @@ extern "C" int kad_lcsa_mask_group(const kad_lcsa_args* a, int count, int emat_d
   KAD_CHECK_ARG(blocks < (1ll << 31), "kad_lcsa_mask_group: too many blocks");
   for (int p = count; p <= KAD_LCSA_GROUP_MAX; ++p) grp.start[p] = (int)blocks;
   hipStream_t st = (hipStream_t)stream;
-  bool one_chunk = true;  // every problem's channels in one 32-channel chunk: the narrow staging
-  for (int p = 0; p < count; ++p) one_chunk = one_chunk && a[p].c <= 32;
-  if (emat_dtype == KAD_F32 && one_chunk)
-    hipLaunchKernelGGL((kad::lcsa_mask_group_kernel<float, 32>), dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
-  else if (emat_dtype == KAD_F32)
-    hipLaunchKernelGGL((kad::lcsa_mask_group_kernel<float, kad::LM_SC>), dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
-  else if (emat_dtype == KAD_F16 && one_chunk)
-    hipLaunchKernelGGL((kad::lcsa_mask_group_kernel<half_t, 32>), dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
+  if (emat_dtype == KAD_F32)
+    hipLaunchKernelGGL(kad::lcsa_mask_group_kernel<float>, dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
   else if (emat_dtype == KAD_F16)
-    hipLaunchKernelGGL((kad::lcsa_mask_group_kernel<half_t, kad::LM_SC>), dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
+    hipLaunchKernelGGL(kad::lcsa_mask_group_kernel<half_t>, dim3((unsigned)blocks), dim3(kad::LM_THREADS), 0, st, grp);
   else
     return fail(KAD_EINVAL, "kad_lcsa_mask_group: emat dtype must be KAD_F32 or KAD_F16");
   return check_launch("kad_lcsa_mask_group");
