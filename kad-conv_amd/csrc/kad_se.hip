@@ -974,6 +974,55 @@ __global__ __launch_bounds__(256) void to_nhwc_v8_kernel(const T* x, T* out, int
   }
 }
 
+// The same for planes of any size: the aligned 16-byte pieces that cover a channel's 64 pixels go to
+// LDS as they lie in memory, and the pixels are read back at the channel's shift (its first pixel's
+// offset from an aligned piece).  Bound by memory; element loads and stores left most of each 64-byte
+// request unused: [8, 256, 50, 50] fp16 12.0 -> 7.1 us (planes of 2500 pixels).
+template <typename T>
+__global__ __launch_bounds__(256) void to_nhwc_shift_kernel(const T* x, T* out, int c, int P, int cs, int npt, int nct,
+                                                            int total, int grid8, int64_t elems) {
+  typedef T v8 __attribute__((ext_vector_type(8)));
+  constexpr int PC = 9, ROW = PC * 8 + 8;  // pieces per channel; 160-byte rows
+  __shared__ __align__(16) T tile[64][ROW];
+  const int bq = (int)(blockIdx.x & 7) * (grid8 >> 3) + (int)(blockIdx.x >> 3);
+  if (bq >= total) return;  // whole block, before the barrier
+  const int pt = bq % npt, r = bq / npt, ct = r % nct, n = r / nct;
+  const int p0 = pt * 64, c0 = ct * 64, tid = threadIdx.x;
+  const int64_t first = ((int64_t)n * c + c0) * P + p0;  // channel c0's first element of the tile
+#pragma unroll
+  for (int u = 0; u < (64 * PC + 255) / 256; ++u) {
+    const int e = tid + 256 * u, cl = e / PC, v = e - cl * PC;
+    if (cl >= 64) continue;
+    const int64_t at = first + (int64_t)cl * P;
+    const int64_t q = (at & ~(int64_t)7) + 8 * v;  // the piece's first element
+    v8 val = {};
+    if (c0 + cl < c && q < at - p0 + P) {  // the piece reaches pixels of the plane
+      if (q + 8 <= elems) {
+        val = *(const v8*)(x + q);
+      } else {
+        for (int j = 0; j < 8; ++j)
+          if (q + j < elems) val[j] = x[q + j];
+      }
+    }
+    *(v8*)&tile[cl][8 * v] = val;
+  }
+  __syncthreads();
+  T* ob = out + (int64_t)n * P * cs;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int pl = tid & 63, g = (tid >> 6) + 4 * u;
+    const int p = p0 + pl, ch = c0 + 8 * g;
+    if (p >= P || ch >= cs) continue;
+    v8 o;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int sh = (int)((first + (int64_t)(8 * g + j) * P) & 7);
+      o[j] = tile[8 * g + j][pl + sh];
+    }
+    *(v8*)(ob + (int64_t)p * cs + ch) = o;
+  }
+}
+
 // ---- channels-last with pixel stride x_cs -> NHWC with channel stride cs (pad channels 0) ----
 // One thread per output piece of 8 channels of one pixel: the input piece is read as
 // elements (x_cs and c need not be multiples of 8), the output written as one vector (16 bytes for 16-bit data).  Consecutive
@@ -1750,10 +1799,17 @@ extern "C" int kad_to_nhwc(const void* x, void* out, int n, int c, int h, int w,
   dim3 grid(ceil_div(P, 64), ceil_div(out_cs, 64), n);
   hipStream_t st = (hipStream_t)stream;
   const int64_t tiles = (int64_t)ceil_div(P, 64) * ceil_div(out_cs, 64) * n;
-  if (dtype != KAD_F32 && P % 8 == 0 && out_cs % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+  if (dtype != KAD_F32 && out_cs % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0 &&
       tiles * 8 < (1ll << 31)) {
     const int npt = ceil_div(P, 64), nct = ceil_div(out_cs, 64), total = (int)tiles, grid8 = round_up(total, 8);
-    if (dtype == KAD_F16)
+    const int64_t elems = (int64_t)n * c * P;
+    if (P % 8 != 0 && dtype == KAD_F16)
+      hipLaunchKernelGGL(to_nhwc_shift_kernel<half_t>, dim3(grid8), dim3(256), 0, st, (const half_t*)x, (half_t*)out,
+                         c, P, out_cs, npt, nct, total, grid8, elems);
+    else if (P % 8 != 0 && dtype == KAD_BF16)
+      hipLaunchKernelGGL(to_nhwc_shift_kernel<bf16_t>, dim3(grid8), dim3(256), 0, st, (const bf16_t*)x, (bf16_t*)out,
+                         c, P, out_cs, npt, nct, total, grid8, elems);
+    else if (dtype == KAD_F16)
       hipLaunchKernelGGL(to_nhwc_v8_kernel<half_t>, dim3(grid8), dim3(256), 0, st, (const half_t*)x, (half_t*)out, c,
                          P, out_cs, npt, nct, total, grid8);
     else if (dtype == KAD_BF16)
