@@ -118,6 +118,13 @@ typedef struct kad_dcn_args {
   float se_inv_count;     /* 1 / (Ho * Wo) */
 } kad_dcn_args;
 
+/* One launch for a deformable convolution's 16-bit operands (dtype KAD_F16 / KAD_BF16): offset32 and
+ * mask32 (n_off / n_mask elements; mask may be NULL) and bias32 ([cout]; bias may be NULL) receive the
+ * values in fp32, wpack what kad_dcn_pack_weights makes of w.  offset32, mask32, wpack 16-byte aligned. */
+int kad_dcn_prep(const void *offset, float *offset32, int64_t n_off, const void *mask, float *mask32, int64_t n_mask,
+                 const void *w, void *wpack, int cin, int cout, const void *bias, float *bias32, int dtype,
+                 void *stream);
+
 /* out = post_scale * act((deform_conv3x3(x, offset, mask, W) + bias) * post_mul + post_add).
  * Stands in for kadc_dcn16.cpp:247-289 `forward*`/`forward_*_unsafe`
  * (kernel kadc_dcn16_kernel.cu:92-314) and for torchvision.ops.deform_conv2d

@@ -144,6 +144,8 @@ SIGNATURES = {
     'kad_pyramid_proj': (c_int, [ctypes.POINTER(PyramidArgs), c_vp]),
     'kad_lcsa_params_elems': (c_i64, [c_int]),
     'kad_lcsa_emat_elems': (c_i64, [c_int]),
+    'kad_dcn_prep': (c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_vp, c_vp, c_int, c_int, c_vp, c_vp, c_int,
+                             c_vp]),
     'kad_axial_sums': (c_int, [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_vp]),
     'kad_axial_sums_nchw': (c_int, [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_int, c_vp]),
     'kad_axial_means': (c_int, [c_vp, c_vp, c_vp, c_int, c_int, c_int, c_int, c_int, c_int, c_vp]),
@@ -337,6 +339,22 @@ def dcn_pack_weights(weight, dtype):
     _check(load().kad_dcn_pack_weights(_ptr(w32), _ptr(out), cin, cout, kad_dtype(dtype), _stream()),
            'kad_dcn_pack_weights')
     return out
+
+
+def dcn_prep(offset, mask, weight, bias):
+    """Contiguous 16-bit tensors of one dtype (mask, bias may be None) -> (offset, mask, bias in fp32,
+    packed weights), as dcn_pack_weights and .float() give them, in one launch."""
+    _need_gpu(offset, mask, weight, bias)
+    cout, cin = weight.shape[:2]
+    if tuple(weight.shape[2:]) != (3, 3):
+        raise ValueError('DSC kernels are 3x3')
+    f32 = [None if t is None else torch.empty(t.shape, dtype=torch.float32, device=t.device)
+           for t in (offset, mask, bias)]
+    wp = torch.empty(dcn_wpack_elems(cin, cout), dtype=weight.dtype, device=weight.device)
+    _check(load().kad_dcn_prep(_ptr(offset), _ptr(f32[0]), offset.numel(), _ptr(mask), _ptr(f32[1]),
+                               0 if mask is None else mask.numel(), _ptr(weight), _ptr(wp), cin, cout, _ptr(bias),
+                               _ptr(f32[2]), kad_dtype(weight.dtype), _stream()), 'kad_dcn_prep')
+    return f32[0], f32[1], f32[2], wp
 
 
 def _set_se_weights(a, se, n, cout, ho, wo):

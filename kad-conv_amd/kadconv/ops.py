@@ -124,11 +124,15 @@ def deform_conv2d(input, offset, weight, bias=None, stride=1, padding=0, dilatio
         return input.new_empty(N, Co, max(Ho, 0), max(Wo, 0))
     x, _ = _nhwc_view(input)
     P = Ho * Wo
-    off = offset.to(torch.float32).contiguous()
-    m = mask.to(torch.float32).contiguous() if mask is not None else None
-    wp = _ext.dcn_pack_weights(weight, dtype)
     b = None
-    if bias is not None:  # fp32 contiguous biases are used as they are (no per-call copy)
+    if dtype != torch.float32 and all(t.dtype == dtype and t.is_contiguous()
+                                      for t in (offset, mask, weight, bias) if t is not None):
+        off, m, b, wp = _ext.dcn_prep(offset, mask, weight, bias)  # one launch instead of five
+    else:
+        off = offset.to(torch.float32).contiguous()
+        m = mask.to(torch.float32).contiguous() if mask is not None else None
+        wp = _ext.dcn_pack_weights(weight, dtype)
+    if bias is not None and b is None:  # fp32 contiguous biases are used as they are (no per-call copy)
         b = bias if (bias.dtype == torch.float32 and bias.is_contiguous()) else bias.detach().float().contiguous()
     out = torch.empty(N, Co, Ho, Wo, dtype=dtype, device=input.device)
     _ext.dcn_fwd(x, C, off, (18 * P, 1, P), m, (9 * P, 1, P), wp, Co, out, stride=s[0], pad=p[0], bias=b,
