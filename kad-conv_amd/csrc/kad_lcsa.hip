@@ -470,8 +470,10 @@ struct LcsaGroup {
   int count;
 };
 
+// Two blocks per CU: at three the fp16 build spills (KAD-Conv branches, [16, 52, 50, 50] 9.0 -> 7.4 us,
+// [4, 96, 75, 75] 6.9 -> 6.1, [16, 36, 100, 100] 17.3 -> 16.8).
 template <typename ET>
-__global__ __launch_bounds__(LM_THREADS, sizeof(ET) == 2 ? 3 : 2) void lcsa_mask_group_kernel(LcsaGroup grp) {
+__global__ __launch_bounds__(LM_THREADS, 2) void lcsa_mask_group_kernel(LcsaGroup grp) {
   const int id = blockIdx.x;
   int p = 0;
 #pragma unroll
