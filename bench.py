@@ -503,7 +503,9 @@ def traffic_from(fetch_csv, write_csv):
                 continue
             name = r['Kernel_Name']
             grid = int(r.get('Grid_Size') or r.get('Grid_Size_X') or 0)
-            kind = 'dsc0' if ('dcn_fwd_kernel' in name or 'dcn_group_kernel' in name) else \
+            # the last two: the names in counter files of earlier trees
+            kind = 'dsc0' if any(k in name for k in ('dg_kernel', 'dg_group_kernel', 'dcn_fwd_kernel',
+                                                     'dcn_group_kernel')) else \
                 'copy' if 'copy' in name.lower() else None
             if kind:
                 rows[kind].append((grid, float(r['Counter_Value'])))
@@ -517,7 +519,7 @@ def traffic_from(fetch_csv, write_csv):
     sf = PROBE_COPY_BYTES / (f['copy'] * 1024.0)
     sw = PROBE_COPY_BYTES / (w['copy'] * 1024.0)
     rd, wr = f['dsc0'] * 1024.0 * sf, w['dsc0'] * 1024.0 * sw
-    out = {'kernel': 'dcn_fwd_kernel<half,half,6,FUSED> branch-0 DSC, [8,86,100,100] fp16',
+    out = {'kernel': 'dg_kernel<half,6,FUSED> branch-0 DSC, [8,86,100,100] fp16',
            'fetch_kib_raw': f['dsc0'], 'write_kib_raw': w['dsc0'],
            'copy_fetch_kib_raw': f['copy'], 'copy_write_kib_raw': w['copy'],
            'fetch_scale': sf, 'write_scale': sw,
@@ -691,12 +693,12 @@ def main():
         if 'dsc' in sd:  # grouped: one launch runs every branch's DSC (+ SE)
             dsc0 = sd['dsc']
             flops = sum(dsc_flops(shape[0], shape[2] >> i, shape[3] >> i, br.c) for i, br in enumerate(plan.branches))
-            kname = ('dcn_group_kernel<half,half,6,FUSED> (the three branches\' DSCs in one launch: conv_offset + '
+            kname = ('dg_group_kernel<half,6,FUSED> (the three branches\' DSCs in one launch: conv_offset + '
                      'DCN + fused SE, c=86/85/85 at 100^2/50^2/25^2, batch 8)')
         else:
             dsc0 = sd['dsc0']
             flops = dsc_flops(shape[0], shape[2], shape[3], plan.branches[0].c)
-            kname = 'dcn_fwd_kernel<half,half,6,FUSED> (branch-0 DSC: conv_offset + DCN, c=86, 8x100x100)'
+            kname = 'dg_kernel<half,6,FUSED> (branch-0 DSC: conv_offset + DCN, c=86, 8x100x100)'
         dcn_us = time_eager(dsc0, args.steps, args.warmup)
         achieved = flops / (dcn_us * 1e-6)
 
