@@ -217,6 +217,10 @@ class KADConvPlan:
         self._lists = {}
         self.groupable = GROUPED and all(br.dsc.use_mask for br in self.branches)
 
+    def __getstate__(self):
+        # recorded launches hold addresses of this plan's own tensors: a copy records its own
+        return dict(self.__dict__, _lists={})
+
     def _grouped(self, x):
         """Grouped launches unless the full-resolution DSC is heavy: N x tiles x 16-channel
         column fragments >= GROUP_MAX_WORK.  Small layers are bound by launch and queue

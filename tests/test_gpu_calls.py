@@ -1,6 +1,8 @@
 """A small KAD-Conv layer's recorded launches (kad_run_calls) against the same stages launched one by
 one: bit for bit, over layouts, channel slices, types and odd sizes, with another input and other
 buffers than those recorded, under graph replay, and with more geometries than a plan keeps."""
+import copy
+
 import pytest
 import torch
 
@@ -70,3 +72,15 @@ def test_recorded_calls_graph_and_bound():
             ref = m(x.clone())
             torch.cuda.synchronize()
             assert torch.equal(y, ref)
+
+
+def test_copied_plan_records_its_own_calls():
+    m = _layer(48, torch.float32)
+    x = _input(1, 48, 9, 12, torch.float32, 'nchw', 0)
+    with torch.no_grad():
+        ref = [m(x) for _ in range(3)][-1]
+        plan = copy.deepcopy(m._kad_plan)
+        assert len(m._kad_plan._lists) == 1 and not plan._lists
+        del m
+        for _ in range(3):
+            assert torch.equal(plan.forward(x), ref)
