@@ -250,7 +250,8 @@ __device__ __forceinline__ typename DcnFrag<T>::frag buf_ld8(__amdgpu_buffer_rsr
 // partials in a fixed order (thread (slice s, channel c) takes tiles s,
 // s + nsl, ...; the slices are then added in order), so the result does not
 // depend on which block came last; then att = sigmoid(W2 relu(W1 g + b1) + b2)
-// with 4 lanes per output and a shuffle reduction.  lds: Cout + hid + THREADS floats.
+// with 4 lanes per output and a shuffle reduction.  lds: Cout + hid + THREADS floats (Cout + hid where one
+// slice takes every tile: its sums are formed in g itself).
 // (dev_load / rmw_store: kad_common.h)
 
 // se_tail_any covers every size; se_tail below the usual ones.
@@ -265,9 +266,9 @@ __device__ __forceinline__ void se_tail_any(const float* __restrict__ partial, c
   const int tid = threadIdx.x;
   float* g = lds;          // [C]
   float* hb = g + C;       // [hid]
-  float* red = hb + hid;   // [nsl][C]
   const float* pn = partial + (int64_t)n * tiles * C;
   const int nsl = C < THREADS ? THREADS / C : 1;
+  float* red = nsl > 1 ? hb + hid : g;  // [nsl][C]: at most THREADS floats behind hb, or g's own
   for (int e = tid; e < nsl * C; e += THREADS) {
     const int s = e / C, ch = e - s * C;
     float acc[4] = {0.f, 0.f, 0.f, 0.f};

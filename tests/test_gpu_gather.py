@@ -95,3 +95,48 @@ def test_se_tail_sizes(c, hid):
         ref = torch.sigmoid(F.linear(torch.relu(F.linear(m, w1.double(), b1.double())), w2.double(), b2.double()))
         assert (att.double().cpu() - ref).abs().max().item() <= 1e-5
     assert (count == 0).all()
+
+
+@pytest.mark.parametrize('dt', ['f16', 'f32'])
+@pytest.mark.parametrize('mode', ['dsc', 'dcn'])
+@pytest.mark.parametrize('c,hid', [(300, 64), (513, 40), (4100, 4100), (4600, 4600), (7000, 16), (11760, 16)])
+def test_se_tail_wide(dt, mode, c, hid):
+    """The general tail of the fused squeeze-excitation, up to the widest layers the entry points take
+    (Cout + hidden + 512 floats in 48 KB): att against the MLP in 64 bits on the mean of the kernel's own
+    output.  Each weight row has 16 nonzeros, half of W1's among the last 64 channels.  Bound: the mean
+    rounded in at most 16 steps, each layer's in at most 24 (adding a zero is exact) on the sums' absolute
+    terms, sigmoid's slope 1 / 4, and 4 units for the sigmoid itself."""
+    from kadconv import _ext
+    dtype = DT[dt]
+    N, C, H, W = 2, 8, 9, 11
+    g = torch.Generator().manual_seed(c + hid)
+    x = torch.randn(N, C, H, W, generator=g)
+    w = torch.randn(c, C, 3, 3, generator=g) / (9 * C) ** 0.5
+    def sparse(rows, cols):
+        at = torch.cat((torch.randint(cols, (rows, 8), generator=g), cols - 1 - torch.randint(min(64, cols), (rows, 8), generator=g)), 1)
+        return torch.zeros(rows, cols).scatter_(1, at, torch.randn(rows, 16, generator=g))
+
+    w1, b1, w2, b2 = sparse(hid, c), torch.randn(hid, generator=g), sparse(c, hid), torch.randn(c, generator=g)
+    print(f'wide se tail {dt} {mode} c={c} hid={hid}', flush=True)
+    att = torch.full((N, c), -1.0, device='cuda')
+    gap = torch.empty(N, _ext.dcn_tiles(H, W), c, device='cuda')
+    out = torch.empty(N, c, H, W, dtype=dtype, device='cuda')
+    kw = dict(out_layout=_ext.KAD_NCHW, gap_partial=gap,
+              se=(w1.cuda(), b1.cuda(), w2.cuda(), b2.cuda(), att, torch.zeros(N, dtype=torch.int32, device='cuda')))
+    xq, wp = nhwc_padded(x.to(dtype).cuda()), _ext.dcn_pack_weights(w.to(dtype).cuda(), dtype)
+    ow = torch.randn(18, C, 3, 3, generator=g) / (9 * C) ** 0.5
+    if mode == 'dsc':
+        _ext.dsc_fwd(xq, C, _ext.dcn_pack_weights(ow.to(dtype).cuda(), dtype), None, None, None, wp, c, out, **kw)
+    else:
+        off = torch.randn(N, H, W, 18, generator=g).cuda()
+        _ext.dcn_fwd(xq, C, off, (H * W * 18, 18, 1), None, None, wp, c, out, **kw)
+    torch.cuda.synchronize()
+    m, u = out.double().cpu().mean((2, 3)), 2.0 ** -24
+    w1, b1, w2, b2 = (t.double() for t in (w1, b1, w2, b2))
+    h = torch.relu(F.linear(m, w1, b1))
+    ref = torch.sigmoid(F.linear(h, w2, b2))
+    em = 16 * u * out.double().abs().cpu().mean((2, 3))
+    eh = F.linear(em, w1.abs()) + 24 * u * (F.linear(m.abs(), w1.abs()) + b1.abs())
+    tol = (F.linear(eh, w2.abs()) + 24 * u * (F.linear(h, w2.abs()) + b2.abs())) / 4 + 4 * u
+    d = (att.double().cpu() - ref).abs()
+    assert (d <= tol).all(), f'max excess {(d - tol).max().item():.2e}, max d {d.max().item():.2e}, tol {tol.max().item():.2e}'

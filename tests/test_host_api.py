@@ -111,3 +111,18 @@ def test_missing_library_raises(monkeypatch, tmp_path):
     monkeypatch.setattr(_ext, '_lib', None)
     with pytest.raises(_ext.KadExtensionError):
         _ext.load()
+
+
+@pytest.mark.parametrize('cout,hid', [(11761, 16), (5888, 5889), (16, 11761)])
+def test_fused_se_past_the_scratch_limit_is_refused(cout, hid):
+    """Cout + hidden + 512 floats past 48 KB: an error from the argument checks, before any launch."""
+    import ctypes
+
+    from kadconv import _ext
+    a = _ext.DcnArgs()
+    a.x = a.wpack = a.off_wpack = a.out = a.offset = a.gap_partial = a.se_w1 = a.se_w2 = a.se_att = a.se_count = 4096
+    a.n, a.cin, a.cout, a.h, a.w, a.stride, a.pad, a.x_cs, a.out_cs = 1, 8, cout, 4, 4, 1, 1, 8, cout
+    a.out_layout, a.dtype, a.se_hid = _ext.KAD_NCHW, _ext.kad_dtype(torch.float16), hid
+    for fn in ('kad_dsc_fwd', 'kad_dcn_fwd'):
+        assert getattr(_ext.load(), fn)(ctypes.byref(a), None) < 0
+        assert b'fused squeeze-excitation: Cout + hidden' in _ext.load().kad_last_error()
