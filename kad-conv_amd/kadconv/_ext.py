@@ -344,8 +344,10 @@ def dcn_pack_weights(weight, dtype):
 def dcn_prep(offset, mask, weight, bias):
     """Contiguous 16-bit tensors of one dtype (mask, bias may be None) -> (offset, mask, bias in fp32,
     packed weights), as dcn_pack_weights and .float() give them, in one launch."""
-    _need_gpu(offset, mask, weight, bias)
     cout, cin = weight.shape[:2]
+    if bias is not None and bias.numel() < cout:
+        raise ValueError(f'bias has {bias.numel()} elements for {cout} output channels')
+    _need_gpu(offset, mask, weight, bias)
     if tuple(weight.shape[2:]) != (3, 3):
         raise ValueError('DSC kernels are 3x3')
     f32 = [None if t is None else torch.empty(t.shape, dtype=torch.float32, device=t.device)

@@ -117,6 +117,8 @@ def deform_conv2d(input, offset, weight, bias=None, stride=1, padding=0, dilatio
         raise ValueError(f'offset shape {tuple(offset.shape)} != {(N, 18, Ho, Wo)} (one offset group)')
     if mask is not None and tuple(mask.shape) != (N, 9, Ho, Wo):
         raise ValueError(f'mask shape {tuple(mask.shape)} != {(N, 9, Ho, Wo)}')
+    if bias is not None and bias.numel() < Co:
+        raise ValueError(f'bias has {bias.numel()} elements for {Co} output channels')
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (input, offset, weight, bias, mask)):
         raise NotImplementedError('kadconv HIP kernels are inference-only (no backward)')
     dtype = input.dtype

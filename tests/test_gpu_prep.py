@@ -30,3 +30,16 @@ def test_dcn_prep(dt, shift, n, cin, cout, h, w, mask, bias):
     assert torch.equal(off32, off.float()) and torch.equal(wp, _ext.dcn_pack_weights(wt, DT[dt]))
     for got, src in ((m32, m), (b32, b)):
         assert got is None if src is None else torch.equal(got, src.float())
+
+
+@pytest.mark.parametrize('dt', ['f16', 'f32'])
+def test_deform_conv2d_bias_length(dt):
+    """A bias shorter than Cout is refused on the device too; one that has more elements uses the first Cout."""
+    import kadconv
+    dtype = {**DT, 'f32': torch.float32}[dt]
+    x, off = torch.randn(1, 8, 5, 6).to('cuda', dtype), torch.randn(1, 18, 5, 6).to('cuda', dtype)
+    w, b = torch.randn(40, 8, 3, 3).to('cuda', dtype), torch.randn(48).to('cuda', dtype)
+    with pytest.raises(ValueError, match='bias has 1 elements for 40'):
+        kadconv.deform_conv2d(x, off, w, b[:1], padding=1)
+    assert torch.equal(kadconv.deform_conv2d(x, off, w, b, padding=1),
+                       kadconv.deform_conv2d(x, off, w, b[:40].contiguous(), padding=1))

@@ -126,3 +126,10 @@ def test_fused_se_past_the_scratch_limit_is_refused(cout, hid):
     for fn in ('kad_dsc_fwd', 'kad_dcn_fwd'):
         assert getattr(_ext.load(), fn)(ctypes.byref(a), None) < 0
         assert b'fused squeeze-excitation: Cout + hidden' in _ext.load().kad_last_error()
+
+
+def test_dcn_prep_rejects_a_short_bias():
+    """kad_dcn_prep reads and writes Cout bias elements."""
+    from kadconv import _ext
+    with pytest.raises(ValueError, match='bias has 3 elements for 4'):
+        _ext.dcn_prep(torch.zeros(1, 18, 5, 5).half(), None, torch.zeros(4, 4, 3, 3).half(), torch.zeros(3).half())
