@@ -14,7 +14,7 @@
 // Modes: EXT    offsets (and mask) come from memory             -> kad_dcn_fwd
 //        FUSED  offsets = conv_offset(x) computed in the block   -> kad_dsc_fwd
 //        PLAIN  ordinary 3x3 convolution (no sampling)          -> kad_conv3x3_fwd, kad_conv_fwd
-// EXT and FUSED run on kad_dcn_gather.h's kernel, at 16-bit Cout <= 16 on dsc2_kernel below; PLAIN on
+// EXT and FUSED run on kad_dcn_gather.h's kernel, narrow 16-bit ones (d2_ok) on dsc2_kernel below; PLAIN on
 // plain_kernel: block = 512 threads (8 waves) x one output tile of up to 128 pixels (TH x TW, chosen
 // per image size to waste few lanes) x 16 NBF output channels; wave w owns tile pixels [16 w, 16 w + 16)
 // and all the block's channels.  Per 32-channel chunk the tile's 3x3 footprint (tile + 1-pixel ring, zero
@@ -402,9 +402,7 @@ __global__ __launch_bounds__(DCN_THREADS, 1) void plain_kernel(kad_dcn_args a, D
 
 // ---- narrow 16-bit DCN / DSC, two or three blocks per CU ------------------------------------------
 // The 16-bit FUSED and EXT paths at stride 1 with up to 16 output channels (KAD-CNet's first-level
-// DSCs).  Against the gathering kernel (us, fp16 DSC alone, this / gathering): Cout 10 at
-// [16, 100, 100] 25 / 36, [8, 100, 100] 15 / 23, [8, 50, 50] 10.6 / 11.3; but Cout 24 at [16, 100, 100]
-// 42 / 37 and Cout 64 85 / 61 (four column fragments): those run there.  Here:
+// DSCs); d2_ok says which of them run here and which on the gathering kernel.  Here:
 //  * 4 waves x 32 pixels (two 16-pixel A fragments per wave): half the weight-fragment reads per
 //    pixel, and they come from global memory (L1 / L2 hits: a column block's packed weights are
 //    at most 9 x 64 x 64 x 2 bytes), so LDS carries only the corner reads;
@@ -1222,9 +1220,18 @@ static int validate_dcn(const kad_dcn_args* a, int mode, DcnGeom* g_out) {
 using namespace kad;
 
 namespace kad {
-// The narrow kernel: 16-bit, stride 1, at most 16 output channels.
-static bool d2_ok(const kad_dcn_args& a) {
-  return (a.dtype == KAD_F16 || a.dtype == KAD_BF16) && a.stride == 1 && a.cout <= 16;
+// The narrow kernel (16-bit, stride 1, at most 16 output channels) or the gathering kernel with 16 columns.
+// The narrow one works in 16-channel half-chunks, the gathering one in 32-channel steps with a cheaper
+// conv_offset, so (us, this / gathering, Cout 16):
+//  * up to 16 input channels here: DSC(16) [16, 100, 100] fp16 25 / 34, deformable part alone 20 / 30;
+//  * DSC of more: there.  32 channels [16, 100, 100] fp16 37 / 34, 64 57 / 48; bf16 128 [8, 25, 25] 35 / 28;
+//  * offsets from memory, an odd count of half-chunks: here.  fp16 48 [8, 100, 100] 25 / 28, 144 49 / 56,
+//    bf16 31 / 32 and 64 / 65; an even count: there.  bf16 64 36 / 31, [8, 25, 25] 17 / 15; fp16 29 / 27, but
+//    above 128 channels of fp16 here again: 256 [8, 100, 100] 74 / 82.
+static bool d2_ok(const kad_dcn_args& a, int mode) {
+  if ((a.dtype != KAD_F16 && a.dtype != KAD_BF16) || a.stride != 1 || a.cout > 16) return false;
+  const int halves = ceil_div(a.cin, 16);
+  return halves == 1 || (mode == MODE_EXT && (halves % 2 == 1 || (a.dtype == KAD_F16 && a.cin > 128)));
 }
 // One region buffer (NRB = 1): a single 16-channel half-chunk, and the conv_offset staging of one
 // 32-channel chunk (footprint and filters, 5 slots per row) and the SE scratch within D2_RBUF.
@@ -1345,7 +1352,7 @@ extern "C" int kad_dcn_fwd(const kad_dcn_args* a, void* stream) {
   int rc = validate_dcn(a, MODE_EXT, &g);
   if (rc) return fail(rc, "kad_dcn_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
-  if (d2_ok(*a)) return dispatch_d2<MODE_EXT>(*a, st, g);
+  if (d2_ok(*a, MODE_EXT)) return dispatch_d2<MODE_EXT>(*a, st, g);
   switch (a->dtype) {
     case KAD_F32: return dcn_gather<float>(*a, g, MODE_EXT, st);
     case KAD_F16: return dcn_gather<half_t>(*a, g, MODE_EXT, st);
@@ -1359,7 +1366,7 @@ extern "C" int kad_dsc_fwd(const kad_dcn_args* a, void* stream) {
   int rc = validate_dcn(a, MODE_FUSED, &g);
   if (rc) return fail(rc, "kad_dsc_fwd: %s", kad_last_error());
   hipStream_t st = (hipStream_t)stream;
-  if (d2_ok(*a)) return dispatch_d2<MODE_FUSED>(*a, st, g);
+  if (d2_ok(*a, MODE_FUSED)) return dispatch_d2<MODE_FUSED>(*a, st, g);
   switch (a->dtype) {
     case KAD_F32: return dcn_gather<float>(*a, g, MODE_FUSED, st);
     case KAD_F16: return dcn_gather<half_t>(*a, g, MODE_FUSED, st);
@@ -1392,7 +1399,7 @@ extern "C" int kad_dsc_fwd_group(const kad_dcn_args* a, int count, void* stream)
   for (int p = count + 1; p <= KAD_DCN_GROUP_MAX; ++p) grp.start[p] = (int)blocks;
   hipStream_t st = (hipStream_t)stream;
   bool all_d2 = true;
-  for (int p = 0; p < count; ++p) all_d2 = all_d2 && d2_ok(a[p]);
+  for (int p = 0; p < count; ++p) all_d2 = all_d2 && d2_ok(a[p], MODE_FUSED);
   if (all_d2) return a[0].dtype == KAD_F16 ? launch_group_d2<half_t>(grp, st) : launch_group_d2<bf16_t>(grp, st);
   switch (a[0].dtype) {
     case KAD_F32: return dcn_gather_group<float>(grp, nbf, st);

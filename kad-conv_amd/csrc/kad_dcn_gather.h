@@ -7,7 +7,8 @@
 //  * Block = 8 waves x one tile of up to 128 output pixels x 16 NBF output channels.  Per k-step the
 //    block builds the sampled tile A [128][64 B] and the weight tile B [16 NBF][64 B] in LDS (both
 //    double-buffered, 16-byte pieces XOR-swizzled by row: a fragment read hits distinct banks) and
-//    multiplies them on MFMA, 4 x 2 waves taking 32 pixels x 8 NBF channels each.
+//    multiplies them on MFMA, 4 x 2 waves taking 32 pixels x 8 NBF channels each (NBF = 1: 8 x 1 waves of
+//    16 pixels; with 32 columns for 16 fp32 DCN 512 -> 16 [8, 25, 25] took 162 us, with 16 126).
 //  * A piece (pixel p, 16 bytes g) belongs to thread 4 p + g: four lanes read one corner's 64
 //    consecutive bytes, which L1 serves as one request (37 TB/s measured over the chip, 8 KB
 //    footprints).  In the MFMA operand's own lane order (16 pixels, then the piece) every lane of a
@@ -71,8 +72,8 @@ template <> struct DgOps<float> {
 };
 
 template <typename T, int NBF, int MODE> struct DgCfg {
-  static_assert(NBF % 2 == 0 && DG_THREADS == 4 * DCN_TILE, "wave grid; one A piece per thread");
-  static constexpr int WCOL = 2, WPX = DG_WAVES / WCOL;          // wave grid: columns x pixels
+  static_assert((NBF == 1 || NBF % 2 == 0) && DG_THREADS == 4 * DCN_TILE, "wave grid; one A piece per thread");
+  static constexpr int WCOL = NBF == 1 ? 1 : 2, WPX = DG_WAVES / WCOL;  // wave grid: columns x pixels
   static constexpr int MF = DCN_TILE / 16 / WPX, NW = NBF / WCOL;
   static constexpr int NB = NBF * 16;
   static constexpr int CH = 64 / (int)sizeof(T);                 // channels per k-step
@@ -551,6 +552,7 @@ static int dg_launch(const kad_dcn_args& a, const DcnGeom& g, int mode, hipStrea
 }
 
 template <typename T> int dcn_gather(const kad_dcn_args& a, const DcnGeom& g, int mode, hipStream_t st) {
+  if (a.cout <= 16) return dg_launch<T, 1>(a, g, mode, st);
   switch (ceil_div(a.cout, 32)) {
     case 1: return dg_launch<T, 2>(a, g, mode, st);
     case 2: return dg_launch<T, 4>(a, g, mode, st);
@@ -565,6 +567,7 @@ template <typename T, int NBF> static int dg_launch_group(const DcnGroup& grp, h
 }
 
 template <typename T> int dcn_gather_group(const DcnGroup& grp, int nbf, hipStream_t st) {
+  if (nbf == 1) return dg_launch_group<T, 1>(grp, st);
   switch ((nbf + 1) / 2) {
     case 1: return dg_launch_group<T, 2>(grp, st);
     case 2: return dg_launch_group<T, 4>(grp, st);

@@ -66,6 +66,16 @@ def test_gather_edges(dt, mode, shape, stride, off_std):
         check_close(out, ref, dtype, f'{dt} {mode} {shape} layout {layout}')
 
 
+@pytest.mark.parametrize('dt', ['f16', 'bf16', 'f32'])
+@pytest.mark.parametrize('mode', ['dsc', 'dcn'])
+@pytest.mark.parametrize('shape', [(2, 16, 16, 13, 21), (1, 17, 1, 9, 10), (2, 24, 15, 17, 11), (1, 33, 16, 12, 25),
+                                   (1, 64, 9, 20, 7), (1, 130, 16, 11, 14), (1, 145, 16, 14, 9)])
+def test_narrow_outputs(dt, mode, shape):
+    """Up to 16 output channels: the narrow kernel and the gathering one with 16 columns, on both sides of
+    the rule between them (half-chunks of 16 input channels, 128 channels)."""
+    test_gather_edges(dt, mode, shape, 1, 2.0)
+
+
 @pytest.mark.parametrize('c,hid', [(10, 32), (16, 16), (40, 40), (86, 86), (90, 91), (128, 128), (85, 7)])
 def test_se_tail_sizes(c, hid):
     """Fused squeeze-excitation with weights that fit the LDS beside the partials and ones that do not
