@@ -11,7 +11,7 @@
 // lane groups' channels on distinct banks).
 // Bound by the matrix cores (157 TFLOP/s) where the grid fills the chip, by the round trips of a step
 // where it does not.  The kernels it replaced loaded single floats, 4 bytes per lane: KAD-CNet-S in
-// fp32, one 512 x 512 image, 10.1 -> 3.3 ms; 1x1 512 -> 512 on [16, 512, 50, 50] runs at 111 TFLOP/s.
+// fp32, one 512 x 512 image, 10.4 -> 3.3 ms; 1x1 512 -> 512 on [16, 512, 50, 50] runs at 111 TFLOP/s.
 #include <type_traits>
 
 #include "kad_common.h"
@@ -33,7 +33,6 @@ struct F32Args {
   int spt, taps;             // k-steps per tap, taps
   int wrow;                  // floats per packed weight row
   int act;                   // KAD_ACT_*
-  int px_tiles;              // per image (conv, NCHW) or over the whole batch (NHWC GEMM)
   int P;                     // output pixels per image, or of the batch
 };
 
@@ -279,18 +278,32 @@ __global__ __launch_bounds__(256, 3) void f32_kernel(F32Args a) {
   else epilogue(std::integral_constant<int, KAD_ACT_NONE>{});
 }
 
+// Time of a launch with B blocks, in tenths of an iteration that has a CU's matrix cores to itself: each block
+// runs its share of the k-steps (two per round of the loop) and about `over` iterations of prologue, sum of the
+// shares and epilogue; a CU's blocks take its matrix cores in turn, and below three of them each one's round
+// trips show.
+static int64_t f32_cost(int64_t B, int iters, int over) {
+  const int64_t q = (B + 255) / 256;  // blocks on the fullest CU
+  return (10 * q + (q == 1 ? 8 : q == 2 ? 4 : 2)) * (round_up(iters, 2) + over);
+}
+
+// The split of k that f32_cost makes fastest.  Over 593 GEMMs and convolutions (8 .. 768 channels, 256 .. 160000
+// pixels, each split timed) its choice is 0.4% off the best on average and 7% at worst; going by block counts
+// alone (512 blocks for KS = 1, then 2) was 13% off, most for one step of channels and for up to 32 columns (us):
+// conv 256 -> 20 [8, 100, 100] 209 -> 126, 40 -> 72 there 87 -> 80, 1x1 16 -> 16 [8, 50, 50] 7.6 -> 4.7.
 template <int MODE>
 static void f32_launch(const F32Args& a, int images, hipStream_t st) {
-  // The split of k by the number of blocks: two 64 x 64 blocks per CU, else two 64 x 32, else 32 x 32.
-  const int ncol = a.colim;
-  const int64_t b1 = (int64_t)images * ceil_div(a.P, 64) * ceil_div(ncol, 64);
-  const int64_t b2 = (int64_t)images * ceil_div(a.P, 64) * ceil_div(ncol, 32);
-  if (b1 >= 512)
-    hipLaunchKernelGGL((f32_kernel<1, MODE>), dim3(ceil_div(a.P, 64), ceil_div(ncol, 64), images), dim3(256), 0, st, a);
-  else if (b2 >= 512)
-    hipLaunchKernelGGL((f32_kernel<2, MODE>), dim3(ceil_div(a.P, 64), ceil_div(ncol, 32), images), dim3(256), 0, st, a);
+  const int ncol = a.colim, steps = a.taps * a.spt;
+  const int p64 = ceil_div(a.P, 64), p32 = ceil_div(a.P, 32), c64 = ceil_div(ncol, 64), c32 = ceil_div(ncol, 32);
+  const int64_t t1 = f32_cost((int64_t)images * p64 * c64, steps, 5);
+  const int64_t t2 = f32_cost((int64_t)images * p64 * c32, ceil_div(steps, 2), 6);
+  const int64_t t4 = f32_cost((int64_t)images * p32 * c32, ceil_div(steps, 4), 8);
+  if (t4 <= t1 && t4 <= t2)
+    hipLaunchKernelGGL((f32_kernel<4, MODE>), dim3(p32, c32, images), dim3(256), 0, st, a);
+  else if (t2 <= t1)
+    hipLaunchKernelGGL((f32_kernel<2, MODE>), dim3(p64, c32, images), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((f32_kernel<4, MODE>), dim3(ceil_div(a.P, 32), ceil_div(ncol, 32), images), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((f32_kernel<1, MODE>), dim3(p64, c64, images), dim3(256), 0, st, a);
 }
 
 int gemm_f32(const kad_gemm_args& a, hipStream_t st) {
@@ -332,6 +345,13 @@ int gemm_f32(const kad_gemm_args& a, hipStream_t st) {
 int conv_f32(const kad_dcn_args& a, int ho, int wo, hipStream_t st) {
   if (a.dtype != KAD_F32 || a.out_layout != KAD_NHWC || a.post_mul || a.post_add || a.post_scale || a.gap_partial ||
       a.n > 65535)
+    return 1;
+  // Up to 16 output channels half of each 32-column tile is empty, and the general kernel computes 16.  It is
+  // the faster one for a single whole 32-channel chunk and where it needs one round of the chip and this one
+  // more (us, this / general): 32 -> 16 [8, 50, 50] 12.3 / 8.6, [16, 100, 100] 40 / 37; 16 -> 16 [8, 50, 50]
+  // 9.5 / 8.7, 64 -> 16 17.5 / 14.2; but [16, 50, 50] 12 / 16 and 25 / 27.
+  if (a.cout <= 16 && ((a.cin > 16 && a.cin <= 32) || (a.n * (int64_t)ceil_div(ho * wo, 64) > 256 &&
+                                                       a.n * (int64_t)kad_dcn_tiles(ho, wo) <= 256)))
     return 1;
   F32Args f{};
   f.x = (const float*)a.x;

@@ -60,3 +60,13 @@ def test_conv3_f32(n, cin, cout, h, w, stride, act):
                   stride=stride, pad=1, bias=b.cuda(), act=code)
     _close(out[..., :cout].permute(0, 3, 1, 2), ref, 'conv')
     assert (out[..., cout:] == 7.0).all()
+
+
+@pytest.mark.parametrize('op', ['gemm', 'conv'])
+@pytest.mark.parametrize('n,cin,cout,h,w', [
+    (1, 16, 16, 50, 50), (2, 512, 20, 40, 41),                          # one k-step; up to 32 columns, many steps
+    (2, 17, 16, 33, 9), (1, 32, 4, 90, 91), (8, 16, 16, 50, 50),        # convolutions of the general kernel
+    (8, 33, 16, 46, 51), (8, 33, 16, 64, 64), (1, 33, 17, 128, 130)])   # and just past its rule
+def test_splits_f32(op, n, cin, cout, h, w):
+    """Both sides of the choice of the split and of the general convolution for up to 16 output channels."""
+    (test_gemm_f32('nchw', n, cin, cout, h, w) if op == 'gemm' else test_conv3_f32(n, cin, cout, h, w, 1, 2))
