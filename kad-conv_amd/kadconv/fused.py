@@ -140,8 +140,18 @@ class DSCPlan:
                                                                  self.cin, h, w, ks, work)))
         b = self.bias if bias is None else bias
         # conv_offset + deformable conv in one kernel: the offsets stay on chip.  Above 128 output channels
-        # every column block forms them again, which still beats a conv_offset launch of its own (fp16 DSC,
-        # one launch / two): [8,256,50,50] 112 / 119 us, [8,256,100,100] 280 / 293, [8,512,25,25] 120 / 135.
+        # every 128-channel column block forms them again: cheaper than a conv_offset launch of its own in 16
+        # bits (us, one launch / two: fp16 256 channels [8, 50, 50] 74 / 76, 512 [8, 25, 25] 82 / 98, bf16 87 / 88
+        # and 103 / 116), dearer in fp32, which is bound by the matrix cores (144 channels [8, 100, 100]
+        # 552 / 520, 256 [8, 50, 50] 385 / 355, 512 [8, 25, 25] 420 / 388, 512 [4, 75, 75] 1147 / 1007).
+        if y.dtype == torch.float32 and self.cout > 128 and se is None:
+            off = torch.empty(n, h, w, 18, dtype=torch.float32, device=dev)
+            st.append(('conv_offset' + tag, lambda: _ext.conv3x3_fwd(y, self.cin, owp, 18, off, bias=self.off_b)))
+            st.append(('dsc' + tag, lambda: _ext.dcn_fwd(
+                y, self.cin, off, (P * 18, 18, 1), mask, (P * 9, 9, 1), wp, self.cout, out, bias=b,
+                post_mul=post_mul, post_add=post_add, post_scale=post_scale, relu=relu, out_layout=out_layout,
+                gap_partial=gap)))
+            return st
         st.append(('dsc' + tag, lambda: _ext.dsc_fwd(
             y, self.cin, owp, self.off_b, mask, (P * 9, 9, 1), wp, self.cout, out, bias=b, post_mul=post_mul,
             post_add=post_add, post_scale=post_scale, relu=relu, out_layout=out_layout, gap_partial=gap, se=se)))

@@ -186,6 +186,25 @@ def test_dsc_config2(dt, C, H):
     check_close(got, O.dsc_forward(sd, '', x.double()), dtype, f'dsc {dt} C={C}')
 
 
+@pytest.mark.parametrize('layout', ['nchw', 'nhwc'])
+@pytest.mark.parametrize('C,split', [(128, False), (130, True)])
+def test_dsc_f32_conv_offset_launch(layout, C, split):
+    """fp32 DSC: above 128 channels conv_offset is a launch of its own."""
+    import kadconv
+    d = kadconv.DSC(C, C)
+    sd = S.make_dsc_state(C, C, seed=C, offset_std_px=2.0)
+    d.load_state_dict(sd, strict=False)
+    d = kadconv.enable_fast_inference(d.to('cuda').eval())
+    x = _x((2, C, 13, 21), torch.float32, seed=C + 1)
+    xd = x.cuda() if layout == 'nchw' else x.cuda().contiguous(memory_format=torch.channels_last)
+    y = torch.zeros(2, 13, 21, (C + 7) // 8 * 8, device='cuda')
+    st = d._kad_plan.stages(y, 2, 13, 21, torch.empty(2, C, 13, 21, device='cuda'), 0)
+    assert any(name == 'conv_offset' for name, _ in st) == split
+    with torch.no_grad():
+        got = d(xd)
+    check_close(got, O.dsc_forward(_sd64(d), '', x.double()), torch.float32, f'dsc f32 C={C} {layout}')
+
+
 @pytest.mark.parametrize('dt,shape', [('f16', (16, 512, 50, 50)), ('f32', (2, 40, 9, 13)),
                                       ('bf16', (3, 72, 20, 21))])
 def test_conv1x1_silu(dt, shape):
