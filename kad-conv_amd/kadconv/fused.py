@@ -231,6 +231,9 @@ class KADConvPlan:
         # recorded launches hold addresses of this plan's own tensors: a copy records its own
         return dict(self.__dict__, _lists={})
 
+    def __setstate__(self, state):
+        self.__dict__.update(state, _lists={})  # also for plans saved without the field
+
     def _grouped(self, x):
         """Grouped launches unless the full-resolution DSC is heavy: N x tiles x 16-channel
         column fragments >= GROUP_MAX_WORK.  Small layers are bound by launch and queue
