@@ -24,6 +24,8 @@ kadc_fused_sm75.py:1400-1488,1544-1557).  Weights are captured when the plan
 is built (as the reference folds BN at patch time, kadc_fused_parallel.py:647-655):
 rebuild it (call enable_fast_inference again) after loading new weights.
 """
+import threading
+
 import torch
 
 from . import _ext
@@ -224,15 +226,25 @@ class KADConvPlan:
             raise NotImplementedError('the fused forward covers n <= 3 branches (the paper uses 3)')
         # grouped: the branches' LCSA and DSC stages run as one launch each (all branches), on the
         # caller's stream; else each branch chain runs on a side stream of its own (see _grouped)
-        self._lists = {}
+        self._lists, self._lists_lock = {}, threading.Lock()
         self.groupable = GROUPED and all(br.dsc.use_mask for br in self.branches)
 
     def __getstate__(self):
         # recorded launches hold addresses of this plan's own tensors: a copy records its own
-        return dict(self.__dict__, _lists={})
+        state = dict(self.__dict__, _lists={})
+        state.pop('_lists_lock')
+        return state
 
     def __setstate__(self, state):
-        self.__dict__.update(state, _lists={})  # also for plans saved without the field
+        self.__dict__.update(state, _lists={}, _lists_lock=threading.Lock())  # also for plans saved without the field
+
+    def _keep(self, key, lst):
+        """Keep lst for the geometry, at most MAX_LISTS of them (several threads may call the layer)."""
+        with self._lists_lock:
+            self._lists.pop(key, None)
+            if len(self._lists) >= MAX_LISTS:
+                del self._lists[next(iter(self._lists))]
+            self._lists[key] = lst
 
     def _grouped(self, x):
         """Grouped launches unless the full-resolution DSC is heavy: N x tiles x 16-channel
@@ -462,12 +474,10 @@ class KADConvPlan:
             st, scratch, out = self._stages_grouped(x, xin, out)
             run = lambda: [fn() for _, fn in st]  # noqa: E731
             if key in self._lists:
-                self._lists[key] = _ext.CallList(run, ([xin], [out_v], scratch))
+                self._keep(key, _ext.CallList(run, ([xin], [out_v], scratch)))
                 return out
             run()
-            if len(self._lists) >= MAX_LISTS:
-                self._lists.pop(next(iter(self._lists)), None)
-            self._lists[key] = None
+            self._keep(key, None)
             return out
         pre, chains, post, out = self.schedule(x, out)
         for _, fn in pre:

@@ -1,11 +1,37 @@
 """KADConvPlan's recorded launches on the host: what a plan keeps per input geometry (no GPU: the launches
 are stubbed)."""
+import sys
+import threading
+
+import torch
+
 import kadconv
+from kadconv import _ext, fused
 from kadconv.fused import KADConvPlan
 
 
 def _plan():
     return KADConvPlan(kadconv.KADConv(24).eval())
+
+
+def _stubbed(monkeypatch):
+    """A plan whose forward does everything but launch, and the geometries it recorded, in order."""
+    plan, recorded = _plan(), []
+
+    class CallList:
+        sizes = [0, 0, 8]
+
+        def __init__(self, run, groups):
+            recorded.append(groups[0][0].shape)
+            run()
+
+        def run(self, *bases):
+            pass
+
+    monkeypatch.setattr(_ext, 'CallList', CallList)
+    monkeypatch.setattr(plan, '_grouped', lambda x: True)
+    monkeypatch.setattr(plan, '_stages_grouped', lambda x, xin, out: ([], [], out))
+    return plan, recorded
 
 
 def test_plan_saved_without_lists_loads():
@@ -16,3 +42,30 @@ def test_plan_saved_without_lists_loads():
     again = KADConvPlan.__new__(KADConvPlan)
     getattr(again, '__setstate__', again.__dict__.update)(state)
     assert again._lists == {} and again.dim == plan.dim
+
+
+def test_lists_with_threads(monkeypatch):
+    """Threads that call one layer with more geometries than it keeps."""
+    plan, _ = _stubbed(monkeypatch)
+    xs = [torch.zeros(1, 24, 4 + k, 4) for k in range(3 * fused.MAX_LISTS)]
+    failed = []
+
+    def work(first):
+        try:
+            for k in range(1500):
+                plan.forward(xs[(first + 7 * k) % len(xs)])
+        except BaseException as e:
+            failed.append(e)
+
+    every = sys.getswitchinterval()
+    sys.setswitchinterval(1e-6)
+    try:
+        threads = [threading.Thread(target=work, args=(11 * t,)) for t in range(8)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        sys.setswitchinterval(every)
+    assert not failed, failed[0]
+    assert len(plan._lists) == fused.MAX_LISTS
