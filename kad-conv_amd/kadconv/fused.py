@@ -238,8 +238,17 @@ class KADConvPlan:
     def __setstate__(self, state):
         self.__dict__.update(state, _lists={}, _lists_lock=threading.Lock())  # also for plans saved without the field
 
+    def _kept(self, key):
+        """The geometry's recorded launches if there are any; it is then the last to be dropped."""
+        with self._lists_lock:
+            lst = self._lists.get(key)
+            if lst is not None:
+                self._lists[key] = self._lists.pop(key)
+            return lst
+
     def _keep(self, key, lst):
-        """Keep lst for the geometry, at most MAX_LISTS of them (several threads may call the layer)."""
+        """Keep lst for the geometry: at most MAX_LISTS, the least recently used one goes (several threads may
+        call the layer)."""
         with self._lists_lock:
             self._lists.pop(key, None)
             if len(self._lists) >= MAX_LISTS:
@@ -463,7 +472,7 @@ class KADConvPlan:
         # later ones replay them as one native call on one workspace (KADConv(64) [1, 64, 80, 80] fp32,
         # eager: 161 -> 65 us per call, 62 of them on the GPU).
         key = (x.shape, x.stride(), x.dtype, x.device, None if out is None else out.stride())
-        lst = self._lists.get(key) if self.groupable else None
+        lst = self._kept(key) if self.groupable else None
         if lst is not None:
             xin, _, out, out_v, _ = self._io(x, out)
             ws = torch.empty(lst.sizes[2], dtype=torch.uint8, device=x.device)

@@ -44,6 +44,19 @@ def test_plan_saved_without_lists_loads():
     assert again._lists == {} and again.dim == plan.dim
 
 
+def test_a_used_list_stays(monkeypatch):
+    """A geometry in use is not dropped for new ones that come and go."""
+    plan, recorded = _stubbed(monkeypatch)
+    hot = torch.zeros(1, 24, 50, 50)
+    for _ in range(3):
+        plan.forward(hot)
+    for k in range(3 * fused.MAX_LISTS):
+        plan.forward(torch.zeros(1, 24, 4 + k, 4))
+        plan.forward(hot)
+    assert recorded.count(hot.shape) == 1
+    assert len(plan._lists) == fused.MAX_LISTS
+
+
 def test_lists_with_threads(monkeypatch):
     """Threads that call one layer with more geometries than it keeps."""
     plan, _ = _stubbed(monkeypatch)
