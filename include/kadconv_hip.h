@@ -552,6 +552,17 @@ typedef struct kad_reloc {
 int kad_run_calls(const void *blob, int64_t blob_bytes, const kad_call *calls, int ncalls, const kad_reloc *relocs,
                   int nrelocs, void *const *bases, int nbases, void *stream);
 
+/* `bytes` bytes at address ptr lie `off` bytes behind bases[base]. */
+typedef struct kad_span {
+  int64_t ptr, bytes, off, base;
+} kad_span;
+
+/* The relocations that move the blob's pointers at the byte offsets `at` from the spans they point into to any
+ * other bases: one for each non-null pointer that starts a span, or else lies in one; others stay as they are.
+ * relocs has room for nat.  Returns their number, or KAD_EINVAL where a pointer fits two spans.  Host only. */
+int kad_find_relocs(const void *blob, int64_t blob_bytes, const int64_t *at, int nat, const kad_span *spans, int nspans,
+                    kad_reloc *relocs);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,4 +1,5 @@
-// kad_run_calls: a layer's launches, prepared once as argument structs, in one host call.
+// kad_run_calls: a layer's launches, prepared once as argument structs, in one host call; kad_find_relocs:
+// which of the structs' pointers move with the caller's tensors.
 #include <string.h>
 
 #include "kad_common.h"
@@ -59,4 +60,35 @@ extern "C" int kad_run_calls(const void* blob, int64_t blob_bytes, const kad_cal
     if (rc) return rc;
   }
   return KAD_OK;
+}
+
+extern "C" int kad_find_relocs(const void* blob, int64_t blob_bytes, const int64_t* at, int nat, const kad_span* spans,
+                               int nspans, kad_reloc* relocs) {
+  KAD_CHECK_ARG((blob || blob_bytes == 0) && (at || nat == 0) && (spans || nspans == 0) && (relocs || nat == 0),
+                "kad_find_relocs: null pointer");
+  KAD_CHECK_ARG(blob_bytes >= 0 && nat >= 0 && nspans >= 0, "kad_find_relocs: negative count");
+  int n = 0;
+  for (int i = 0; i < nat; ++i) {
+    KAD_CHECK_ARG(at[i] >= 0 && at[i] + 8 <= blob_bytes, "kad_find_relocs: pointer %d outside the blob", i);
+    int64_t p;
+    memcpy(&p, (const char*)blob + at[i], sizeof(p));
+    if (!p) continue;
+    int start = 0, inside = 0;  // spans that begin at p, that hold it
+    const kad_span *s0 = nullptr, *s1 = nullptr;
+    for (int k = 0; k < nspans; ++k) {
+      const kad_span& s = spans[k];
+      if (p == s.ptr && s.bytes > 0) {
+        ++start;
+        s0 = &s;
+      } else if (p > s.ptr && p < s.ptr + s.bytes) {
+        ++inside;
+        s1 = &s;
+      }
+    }
+    // two channel slices of one buffer span each other's starts: a start decides
+    KAD_CHECK_ARG(start <= 1 && (start == 1 || inside <= 1), "kad_find_relocs: pointer %d fits two spans", i);
+    const kad_span* s = start ? s0 : s1;
+    if (s) relocs[n++] = {at[i], s->off + (p - s->ptr), (int)s->base};
+  }
+  return n;
 }

@@ -10,7 +10,7 @@ Every wrapper takes torch tensors, checks device/dtype/contiguity on the host,
 passes raw pointers plus ``torch.cuda.current_stream()`` and converts a
 negative return code into ``RuntimeError`` carrying ``kad_last_error()``.
 """
-import bisect
+import array
 import ctypes
 import functools
 import threading
@@ -125,6 +125,7 @@ SIGNATURES = {
     'kad_abi_version': (c_int, []),
     'kad_last_error': (ctypes.c_char_p, []),
     'kad_run_calls': (c_int, [c_vp, c_i64, c_vp, c_int, c_vp, c_int, c_vp, c_int, c_vp]),
+    'kad_find_relocs': (c_int, [c_vp, c_i64, c_vp, c_int, c_vp, c_int, c_vp]),
     'kad_dcn_wpack_elems': (c_i64, [c_int, c_int]),
     'kad_dcn_pack_weights': (c_int, [c_vp, c_vp, c_int, c_int, c_int, c_vp]),
     'kad_dcn_tiles': (c_int, [c_int, c_int]),
@@ -219,7 +220,7 @@ def _stream():
 
 
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def kad_dtype(dtype):
@@ -237,7 +238,7 @@ def _need_gpu(*ts):
 
 # ---------------------------------------------------------------------------- recorded calls
 class _Recorder(threading.local):
-    calls = None    # while recording: [(CALL_*, [argument structs], int argument)]
+    calls = None    # while a CallList records: [(CALL_*, argument struct or array of them, int argument)]
 
 
 _rec = _Recorder()
@@ -245,27 +246,37 @@ _rec = _Recorder()
 
 def _note(fn, structs, arg=0):
     if _rec.calls is not None:
-        _rec.calls.append((fn, list(structs), arg))
+        _rec.calls.append((fn, structs, arg))
 
 
-@functools.lru_cache(maxsize=None)
 def _pointer_offsets(cls):
-    """Byte offsets of the pointer fields (and of pointer arrays' elements) of an argument struct."""
-    offs = []
-    for name, typ in cls._fields_:
-        at = getattr(cls, name).offset
-        if typ is c_vp:
-            offs.append(at)
-        elif issubclass(typ, ctypes.Array) and typ._type_ is c_vp:
-            offs += [at + 8 * i for i in range(typ._length_)]
-    return tuple(offs)
+    """Byte offsets of the pointer fields of an argument struct (or array of structs)."""
+    if issubclass(cls, ctypes.Array):
+        step = ctypes.sizeof(cls._type_)
+        return [i * step + off for i in range(cls._length_)
+                for off in ([0] if cls._type_ is c_vp else _pointer_offsets(cls._type_))]
+    return [getattr(cls, name).offset + off for name, typ in cls._fields_
+            for off in ([0] if typ is c_vp else _pointer_offsets(typ) if issubclass(typ, ctypes.Array) and
+                        typ._type_ is c_vp else [])]
+
+
+@functools.lru_cache(maxsize=64)
+def _call_layout(kinds):
+    """(kad_call array, byte offsets of the blob's pointers) for calls of ((CALL_*, struct type, argument), ..)."""
+    calls, at, pointers = [], 0, []
+    for fn, cls, arg in kinds:
+        calls.append(Call(fn, cls._length_ if issubclass(cls, ctypes.Array) else 1, at, arg))
+        pointers += [at + off for off in _pointer_offsets(cls)]
+        at += ctypes.sizeof(cls)
+    return (Call * len(calls))(*calls), array.array('q', pointers)
 
 
 class CallList:
     """The calls that `run` makes, as argument structs for kad_run_calls: one host call instead of one
     per launch.  Their pointers into `groups` (base i: the tensors of groups[i], laid out one behind the
     other at 256-byte steps when a group has several) become offsets from that base; every other pointer
-    belongs to the caller's long-lived tensors and stays.  Nothing else of the recorded run is kept."""
+    belongs to the caller's long-lived tensors and stays.  Nothing else of the recorded tensors is kept.
+    `movable` is False where tensors of two groups cannot be told apart (they start at one address)."""
 
     def __init__(self, run, groups):
         _rec.calls = []
@@ -279,32 +290,24 @@ class CallList:
             at = 0
             for t in tensors:
                 # extent of the view's storage span (a channel slice spans more than its elements)
-                n = (sum((d - 1) * s for d, s in zip(t.shape, t.stride())) + 1) * t.element_size()
-                p = t.data_ptr()
-                spans.append((p, p + n, base, at - p))
+                n = t.nbytes if t.is_contiguous() else \
+                    (sum((d - 1) * s for d, s in zip(t.shape, t.stride())) + 1) * t.element_size()
+                spans += (t.data_ptr(), n, at, base)
                 at += (n + 255) // 256 * 256
             self.sizes.append(at)
-        spans.sort()
-        starts = [sp[0] for sp in spans]
-        blob, relocs, cl = bytearray(), [], []
-        for fn, structs, arg in calls:
-            cl.append(Call(fn, len(structs), len(blob), arg))
-            for st in structs:
-                raw = bytes(st)
-                for off in _pointer_offsets(type(st)):
-                    v = int.from_bytes(raw[off:off + 8], 'little')
-                    k = bisect.bisect_right(starts, v) - 1
-                    if v and k >= 0 and v < spans[k][1]:
-                        relocs.append(Reloc(len(blob) + off, v + spans[k][3], spans[k][2]))
-                blob += raw
-        self._blob = ctypes.create_string_buffer(bytes(blob), len(blob))
-        self._calls = (Call * len(cl))(*cl)
-        self._relocs = (Reloc * len(relocs))(*relocs)
-        self._args = (ctypes.addressof(self._blob), len(blob), ctypes.addressof(self._calls), len(cl),
-                      ctypes.addressof(self._relocs), len(relocs))
+        self._calls, pointers = _call_layout(tuple([(fn, type(st), arg) for fn, st, arg in calls]))
+        self._blob = b''.join([bytes(st) for _, st, _ in calls])
+        self._relocs = (Reloc * len(pointers))()
+        where, spans = pointers.buffer_info()[0], array.array('q', spans)
+        n = load().kad_find_relocs(self._blob, len(self._blob), where, len(pointers), spans.buffer_info()[0],
+                                   len(spans) // 4, self._relocs)
+        self.movable = n >= 0
+        self._args = (self._blob, len(self._blob), self._calls, len(self._calls))
+        self._moves = (self._relocs, n)
 
     def run(self, *bases):
-        _check(load().kad_run_calls(*self._args, (c_vp * len(bases))(*bases), len(bases), _stream()), 'kad_run_calls')
+        _check(load().kad_run_calls(*self._args, *self._moves, (c_vp * len(bases))(*bases), len(bases), _stream()),
+               'kad_run_calls')
 
 
 # ---------------------------------------------------------------------------- DCN
@@ -467,7 +470,7 @@ def dsc_fwd(x_nhwc, cin, off_wpack, off_bias, mask, mask_strides, wpack, cout, o
 def dsc_fwd_group(args):
     """Several fused DSC problems (kad_dcn_args from dsc_args) in one launch."""
     arr = (DcnArgs * len(args))(*args)
-    _note(CALL_DSC, args)
+    _note(CALL_DSC, arr)
     _check(load().kad_dsc_fwd_group(arr, len(args), _stream()), 'kad_dsc_fwd_group')
 
 
@@ -483,13 +486,13 @@ def lcsa_args(rows, nrp, cols, ncp, arow, colm, params, emat, ebias, mask, n, c,
 
 def lcsa_prep_group(args):
     arr = (LcsaArgs * len(args))(*args)
-    _note(CALL_LCSA_PREP, args)
+    _note(CALL_LCSA_PREP, arr)
     _check(load().kad_lcsa_prep_group(arr, len(args), _stream()), 'kad_lcsa_prep_group')
 
 
 def lcsa_mask_group(args, emat_dtype):
     arr = (LcsaArgs * len(args))(*args)
-    _note(CALL_LCSA_MASK, args, kad_dtype(emat_dtype))
+    _note(CALL_LCSA_MASK, arr, kad_dtype(emat_dtype))
     _check(load().kad_lcsa_mask_group(arr, len(args), kad_dtype(emat_dtype), _stream()), 'kad_lcsa_mask_group')
 
 
@@ -562,6 +565,7 @@ def kaddown_prep(x, u, nb):
 
 
 # ---------------------------------------------------------------------------- pyramid
+@functools.lru_cache(maxsize=256)
 def pyramid_tiles(h, w):
     tx, ty = c_int(), c_int()
     _check(load().kad_pyramid_tiles(h, w, ctypes.byref(tx), ctypes.byref(ty)), 'kad_pyramid_tiles')
@@ -595,7 +599,7 @@ def pyramid_proj(x, in_layout, cin, branches):
         a.cout[i], a.out_cs[i], a.out_h[i], a.out_w[i] = b['cout'], out.shape[3], out.shape[1], out.shape[2]
         a.rowpart[i] = b['rowpart'].data_ptr() if b.get('rowpart') is not None else None
         a.colpart[i] = b['colpart'].data_ptr() if b.get('colpart') is not None else None
-    _note(CALL_PYRAMID, [a])
+    _note(CALL_PYRAMID, a)
     _check(load().kad_pyramid_proj(ctypes.byref(a), _stream()), 'kad_pyramid_proj')
 
 
@@ -797,8 +801,8 @@ def scale_residual(out, att, residual, c_off, c, layout):
         raise ValueError('scale_residual wants dense out / residual of one shape')
     if att.dtype != torch.float32 or tuple(att.shape) != (N, c):
         raise TypeError('att must be float32 [N, c]')
-    _note(CALL_SCALE_RESIDUAL, [ScaleArgs(_ptr(out), _ptr(att), _ptr(residual), N, c, H, W, C, c_off, layout,
-                                          kad_dtype(out.dtype))])
+    _note(CALL_SCALE_RESIDUAL, ScaleArgs(_ptr(out), _ptr(att), _ptr(residual), N, c, H, W, C, c_off, layout,
+                                         kad_dtype(out.dtype)))
     _check(load().kad_scale_residual(_ptr(out), _ptr(att), _ptr(residual), N, c, H, W, C, c_off, layout,
                                      kad_dtype(out.dtype), _stream()), 'kad_scale_residual')
     return out
@@ -835,7 +839,7 @@ def branch_merge(out, layout, branches, residual=None, gate=None, channels=None)
         _, zh, zw, zcs = _nhwc_cs(z)   # z may be a channel slice (e.g. the output's own window)
         a.br_h[i], a.br_w[i], a.br_cs[i] = zh, zw, zcs
         a.br_coeff[i] = float(b.get('coeff', 1.0))
-    _note(CALL_MERGE, [a])
+    _note(CALL_MERGE, a)
     _check(load().kad_branch_merge(ctypes.byref(a), _stream()), 'kad_branch_merge')
     return out
 

@@ -241,9 +241,9 @@ class KADConvPlan:
     def _kept(self, key):
         """The geometry's recorded launches if there are any; it is then the last to be dropped."""
         with self._lists_lock:
-            lst = self._lists.get(key)
+            lst = self._lists.pop(key, None)
             if lst is not None:
-                self._lists[key] = self._lists.pop(key)
+                self._lists[key] = lst
             return lst
 
     def _keep(self, key, lst):
@@ -322,7 +322,16 @@ class KADConvPlan:
         in_layout = out_layout = _ext.KAD_NHWC if _channels_last_view(x) else _ext.KAD_NCHW
         out_v = out.permute(0, 2, 3, 1) if out_layout == _ext.KAD_NHWC else out
         ntx, nty = _ext.pyramid_tiles(H, W)
-        pyr, lcsa, dcn, keep, merges = [], [], {}, [], []
+        # the fp32 scratch of all branches in one allocation (a tensor each cost the host 25 us a call)
+        sizes = []
+        for i, br in enumerate(self.branches):
+            h, w = H >> i, W >> i
+            sizes += (N * ntx * h * br.c, N * nty * w * br.c, N * h * br.c, N * w * br.c, N * h * w * 9,
+                      N * _ext.dcn_tiles(h, w) * br.c)
+        sizes = [(s + 63) // 64 * 64 for s in sizes]  # 256-byte steps
+        ws = torch.empty(sum(sizes), dtype=torch.float32, device=dev)
+        parts = iter(ws.split(sizes))
+        pyr, lcsa, dcn, keep, merges = [], [], {}, [ws], []
         edt = _emat_dtype(dtype)
         st = []
         for i, br in enumerate(self.branches):
@@ -330,17 +339,12 @@ class KADConvPlan:
             P = h * w
             full = (h, w) == (H, W)
             y = torch.empty(N, h, w, br.cs, dtype=dtype, device=dev)
-            rows = torch.empty(N, ntx, h, br.c, dtype=torch.float32, device=dev)
-            cols = torch.empty(N, nty, w, br.c, dtype=torch.float32, device=dev)
+            rows, cols, arow, colm, mask, gap = [next(parts) for _ in range(6)]
             pyr.append({'wpack': br.proj_packed(dtype), 'bias': br.proj_b, 'cout': br.c, 'out': y,
                         'rowpart': rows, 'colpart': cols})
             wp, owp, emat, ebias = br.dsc.packed(dtype)
-            arow = torch.empty(N, h, br.c, dtype=torch.float32, device=dev)
-            colm = torch.empty(N, w, br.c, dtype=torch.float32, device=dev)
-            mask = torch.empty(N, h, w, 9, dtype=torch.float32, device=dev)
             lcsa.append(_ext.lcsa_args(rows, ntx, cols, nty, arow, colm, br.dsc.lcsa, emat, ebias, mask, N, br.c, h,
                                        w))
-            gap = torch.empty(N, _ext.dcn_tiles(h, w), br.c, dtype=torch.float32, device=dev)
             if full:  # written straight into its channel slice of the output
                 z = out_v[:, br.c_off:br.c_off + br.c] if out_layout == _ext.KAD_NCHW \
                     else out_v[..., br.c_off:br.c_off + br.c]
@@ -354,9 +358,9 @@ class KADConvPlan:
                               post_mul=br.bn_a, post_add=br.bn_b, post_scale=br.scale, relu=True,
                               out_layout=z_layout, gap_partial=gap, se=se)
             dcn.setdefault(min((br.c + 15) // 16, 8), []).append(a)   # one launch per instantiation
-            keep += [y, rows, cols, arow, colm, mask, gap, att] + ([] if full else [z])
+            keep += [y, att] if full else [y, att, z]
             merges.append((full, {'z': z, 'c': br.c, 'c_off': br.c_off, 'att': att}))
-        st.append(('pyramid', lambda: _ext.pyramid_proj(xin, in_layout, C, pyr)))
+        st.append(('pyramid', lambda keep=keep: _ext.pyramid_proj(xin, in_layout, C, pyr)))
         st.append(('lcsa_prep', lambda keep=keep: _ext.lcsa_prep_group(lcsa)))
         st.append(('lcsa_mask', lambda keep=keep: _ext.lcsa_mask_group(lcsa, edt)))
         for k, args in dcn.items():
@@ -468,9 +472,10 @@ class KADConvPlan:
         stream, the branch chains forked onto side streams (concurrent on the GPU;
         HIP-graph capture records the fork/join as graph edges), merge after the join.
         out: see _io (channels-last input only)."""
-        # A small layer's launches cost the host more than the GPU: a geometry's second call records them,
-        # later ones replay them as one native call on one workspace (KADConv(64) [1, 64, 80, 80] fp32,
-        # eager: 161 -> 65 us per call, 62 of them on the GPU).
+        # A small layer's launches cost the host more than the GPU: a geometry's first call records them (while
+        # the GPU works), later ones replay them as one native call on one workspace.  KADConv(64) fp32, called
+        # directly, us: [1, 64, 80, 80] 161 -> 65 per replay, 62 of them on the GPU; a map seen for the first time
+        # 182 -> 175, for the second 180 -> 98 (waited for each).
         key = (x.shape, x.stride(), x.dtype, x.device, None if out is None else out.stride())
         lst = self._kept(key) if self.groupable else None
         if lst is not None:
@@ -481,12 +486,9 @@ class KADConvPlan:
         if self._grouped(x):
             xin, _, out, out_v, _ = self._io(x, out)
             st, scratch, out = self._stages_grouped(x, xin, out)
-            run = lambda: [fn() for _, fn in st]  # noqa: E731
-            if key in self._lists:
-                self._keep(key, _ext.CallList(run, ([xin], [out_v], scratch)))
-                return out
-            run()
-            self._keep(key, None)
+            lst = _ext.CallList(lambda: [fn() for _, fn in st], ([xin], [out_v], scratch))
+            if lst.movable:
+                self._keep(key, lst)
             return out
         pre, chains, post, out = self.schedule(x, out)
         for _, fn in pre:

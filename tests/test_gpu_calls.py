@@ -39,7 +39,7 @@ def test_recorded_calls_match_stages(dt, layout, dim, n, h, w):
     plan = m._kad_plan
     print(f'calls {dt} {layout} {dim, n, h, w}', flush=True)
     with torch.no_grad():
-        keep = [m(_input(n, dim, h, w, DT[dt], layout, 0)) for _ in range(2)]  # runs, then records
+        keep = [m(_input(n, dim, h, w, DT[dt], layout, 0)) for _ in range(2)]  # records, then replays
         assert [v is not None for v in plan._lists.values()] == [True]
         for seed in (1, 2):
             x = _input(n, dim, h, w, DT[dt], layout, seed)
@@ -84,3 +84,37 @@ def test_copied_plan_records_its_own_calls():
         del m
         for _ in range(3):
             assert torch.equal(plan.forward(x), ref)
+
+
+@pytest.mark.parametrize('dt', ['f32', 'f16', 'bf16'])
+@pytest.mark.parametrize('dim,n,h,w', [(48, 2, 21, 37), (130, 1, 20, 12)])
+@pytest.mark.parametrize('place', ['x first', 'out first', 'two buffers'])
+def test_recorded_calls_with_out(dt, dim, n, h, w, place):
+    """forward(x, out=) on channel slices, x and out of one wide buffer (the detector's concats) or of two:
+    every call on buffers of its own, bit for bit as the stages one by one; nothing else is written."""
+    dtype, cs = DT[dt], (dim + 7) // 8 * 8
+    plan = _layer(dim, dtype)._kad_plan
+    wide = 2 * cs + 24
+    ax, ao = {'x first': (8, cs + 16), 'out first': (cs + 16, 8), 'two buffers': (8, 16)}[place]
+    print(f'calls out {dt} {dim, n, h, w} {place}', flush=True)
+
+    def buffers(seed):
+        g = torch.Generator().manual_seed(seed)
+        bx = torch.randn(n, h, w, wide, generator=g).to('cuda', dtype)
+        bo = bx if place != 'two buffers' else torch.randn(n, h, w, wide, generator=g).to('cuda', dtype)
+        return bx, bo, bx[..., ax:ax + dim].permute(0, 3, 1, 2), bo[..., ao:ao + dim].permute(0, 3, 1, 2)
+
+    past = []
+    with torch.no_grad():
+        for seed in range(4):
+            bx, bo, x, out = buffers(seed)
+            rx, ro, x2, out2 = buffers(seed)
+            st, _ = plan.schedule_grouped(x2, out2)
+            for _, fn in st:
+                fn()
+            assert plan.forward(x, out=out) is out
+            assert torch.equal(bx, rx) and torch.equal(bo, ro)   # the slices and all around them
+            past.append((bx, bo, bx.clone(), bo.clone()))
+        assert len(plan._lists) == 1
+        for bx, bo, cx, co in past:
+            assert torch.equal(bx, cx) and torch.equal(bo, co)

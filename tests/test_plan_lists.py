@@ -19,11 +19,10 @@ def _stubbed(monkeypatch):
     plan, recorded = _plan(), []
 
     class CallList:
-        sizes = [0, 0, 8]
+        sizes, movable = [0, 0, 8], True
 
         def __init__(self, run, groups):
             recorded.append(groups[0][0].shape)
-            run()
 
         def run(self, *bases):
             pass
@@ -55,6 +54,19 @@ def test_a_used_list_stays(monkeypatch):
         plan.forward(hot)
     assert recorded.count(hot.shape) == 1
     assert len(plan._lists) == fused.MAX_LISTS
+
+
+def test_first_call_records(monkeypatch):
+    """A geometry is prepared once, on its first call; one whose pointers cannot be told apart, each time."""
+    plan, recorded = _stubbed(monkeypatch)
+    x = torch.zeros(1, 24, 6, 4)
+    for _ in range(3):
+        plan.forward(x)
+    assert len(recorded) == 1 and len(plan._lists) == 1
+    monkeypatch.setattr(_ext.CallList, 'movable', False)
+    for _ in range(3):
+        plan.forward(x.new_zeros(1, 24, 7, 4))
+    assert len(recorded) == 4 and len(plan._lists) == 1
 
 
 def test_lists_with_threads(monkeypatch):
