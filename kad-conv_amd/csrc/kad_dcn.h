@@ -53,47 +53,13 @@ inline DcnGeom make_geom(const kad_dcn_args& a, int ho, int wo, int tile = DCN_T
   return g;
 }
 
-// ---- sample info ----------------------------------------------------------------------------
-// Fast-path record per (tap, pixel): byte offsets of the four corners inside the
-// staged region and the corner weights (16-bit paths: 16-bit offsets, fp16
-// weights; fp32 path: 32-bit offsets, fp32 weights).  Samples that are dead
-// (all weights 0) or outside a capped region get zero weights here; the latter
-// are accumulated by a separate pass from global memory (s_slow).
-struct __align__(16) Info16 { unsigned o01, o23; unsigned w01, w23; };  // weights as 2 x half2
-struct __align__(16) Info32 { unsigned o[4]; float w[4]; };
-
+// ---- samples ----------------------------------------------------------------------------------
+// The kernels keep a record per (tap, pixel) in LDS: where its top-left corner lies, the corner steps, and
+// the four corner weights times the mask (sample_geom), in 16-bit paths as fp16: uint2 {w00 | w01, w10 | w11}.
 __device__ __forceinline__ unsigned pack_h2(float a, float b) {
   const half2_t h{(half_t)a, (half_t)b};
   return __builtin_bit_cast(unsigned, h);
 }
-
-template <typename T> struct InfoOf { typedef Info16 type; };
-template <> struct InfoOf<float> { typedef Info32 type; };
-
-template <typename T>
-__device__ __forceinline__ typename InfoOf<T>::type make_info(const unsigned* o, const float* w) {
-  typename InfoOf<T>::type r;
-  if constexpr (sizeof(T) == 4) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      r.o[i] = o[i];
-      r.w[i] = w[i];
-    }
-  } else {
-    r.o01 = o[0] | (o[1] << 16);
-    r.o23 = o[2] | (o[3] << 16);
-    r.w01 = pack_h2(w[0], w[1]);
-    r.w23 = pack_h2(w[2], w[3]);
-  }
-  return r;
-}
-
-// byte offset of corner j of a record
-__device__ __forceinline__ unsigned corner(const Info16& in, int j) {
-  const unsigned v = j < 2 ? in.o01 : in.o23;
-  return (j & 1) ? v >> 16 : v & 0xffffu;
-}
-__device__ __forceinline__ unsigned corner(const Info32& in, int j) { return in.o[j]; }
 
 // ---- A fragment from four corners ------------------------------------------------------------
 template <typename T> struct DcnFrag;
@@ -101,8 +67,8 @@ template <typename T> struct DcnFrag;
 template <> struct DcnFrag<half_t> {
   typedef half8_t frag;
   static __device__ __forceinline__ frag blend(const half8_t& v0, const half8_t& v1, const half8_t& v2,
-                                               const half8_t& v3, const Info16& in) {
-    const half2_t w01 = __builtin_bit_cast(half2_t, in.w01), w23 = __builtin_bit_cast(half2_t, in.w23);
+                                               const half8_t& v3, const uint2& w) {
+    const half2_t w01 = __builtin_bit_cast(half2_t, w.x), w23 = __builtin_bit_cast(half2_t, w.y);
     frag r = v0 * w01[0];
     r += v1 * w01[1];
     r += v2 * w23[0];
@@ -117,8 +83,8 @@ template <> struct DcnFrag<half_t> {
 template <> struct DcnFrag<bf16_t> {
   typedef bf16x8_t frag;
   static __device__ __forceinline__ frag blend(const bf16x8_t& v0, const bf16x8_t& v1, const bf16x8_t& v2,
-                                               const bf16x8_t& v3, const Info16& in) {
-    const half2_t w01 = __builtin_bit_cast(half2_t, in.w01), w23 = __builtin_bit_cast(half2_t, in.w23);
+                                               const bf16x8_t& v3, const uint2& w) {
+    const half2_t w01 = __builtin_bit_cast(half2_t, w.x), w23 = __builtin_bit_cast(half2_t, w.y);
     const float a = (float)w01[0], b = (float)w01[1], c = (float)w23[0], d = (float)w23[1];
     frag r;
 #pragma unroll
@@ -135,13 +101,6 @@ struct f32x8 { floatx4 lo, hi; };
 
 template <> struct DcnFrag<float> {
   typedef f32x8 frag;
-  static __device__ __forceinline__ frag blend(const f32x8& v0, const f32x8& v1, const f32x8& v2,
-                                               const f32x8& v3, const Info32& in) {
-    frag r;
-    r.lo = v0.lo * in.w[0] + v1.lo * in.w[1] + v2.lo * in.w[2] + v3.lo * in.w[3];
-    r.hi = v0.hi * in.w[0] + v1.hi * in.w[1] + v2.hi * in.w[2] + v3.hi * in.w[3];
-    return r;
-  }
   // 8 MFMA steps of k=4: step j consumes slot j of every lane group, i.e.
   // k = 8 * group + j on both operands.
   static __device__ __forceinline__ floatx4 mma(const frag& a, const frag& b, floatx4 c) {
@@ -219,8 +178,6 @@ __device__ __forceinline__ void sample_geom(float py, float px, float m, int h, 
 // size, so pieces outside the image (padding ring, channels past Cin, unused
 // staging slots) are staged as zeros with no branch; per-thread byte offsets are
 // computed once per block and only shifted per channel chunk.
-constexpr uint32_t DCN_OOB = KAD_OOB;
-
 template <typename T>
 __device__ __forceinline__ typename DcnFrag<T>::frag buf_ld8(__amdgpu_buffer_rsrc_t r, uint32_t voff) {
   typedef typename DcnFrag<T>::frag F;
@@ -431,8 +388,7 @@ struct DcnGroup {
   int count;
 };
 
-// kad_dcn_gather.h's kernels, one translation unit per data type: 1 when they do not take the launch,
-// else 0 or a KAD_E* code.
+// kad_dcn_gather.h's kernels, one translation unit per data type: 0 or a KAD_E* code.
 template <typename T> int dcn_gather(const kad_dcn_args& a, const DcnGeom& g, int mode, hipStream_t st);
 template <typename T> int dcn_gather_group(const DcnGroup& grp, int nbf, hipStream_t st);
 

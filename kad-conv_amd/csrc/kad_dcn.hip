@@ -72,14 +72,14 @@ template <typename T, int CAP> struct RegionTile {
   static constexpr int RPT = (CAP + DCN_SLOT - 1) / DCN_SLOT;
   static constexpr bool RAGGED = CAP % DCN_SLOT != 0;
   typename DcnFrag<T>::frag v[RPT];
-  uint32_t voff[RPT];  // byte offset of the piece's chunk-0 channels in the image, or DCN_OOB
+  uint32_t voff[RPT];  // byte offset of the piece's chunk-0 channels in the image, or KAD_OOB
   // npix = rows x cols pixels starting at (y0, x0); parts outside the image read 0
   __device__ __forceinline__ void setup(int y0, int x0, int cols, int npix, float inv_cols, int h, int w, int x_cs,
                                         int tid) {
 #pragma unroll
     for (int u = 0; u < RPT; ++u) {
       const int q = (tid >> 2) + u * DCN_SLOT;
-      uint32_t o = DCN_OOB;
+      uint32_t o = KAD_OOB;
       if (q < npix) {
         const int qy = (int)(((float)q + 0.5f) * inv_cols);
         const int gy = y0 + qy, gx = x0 + q - qy * cols;
@@ -93,7 +93,7 @@ template <typename T, int CAP> struct RegionTile {
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t r, int c, bool chs_ok) {
     const uint32_t cofs = (uint32_t)(c * 32 * (int)sizeof(T));
 #pragma unroll
-    for (int u = 0; u < RPT; ++u) v[u] = buf_ld8<T>(r, chs_ok ? voff[u] + cofs : DCN_OOB);
+    for (int u = 0; u < RPT; ++u) v[u] = buf_ld8<T>(r, chs_ok ? voff[u] + cofs : KAD_OOB);
   }
   __device__ __forceinline__ void store(T* region, int pxs, int tid) {
     T* base = region + (tid >> 2) * pxs + (tid & 3) * 8;
@@ -114,7 +114,7 @@ template <typename T, int NBC> struct WeightTile {
 #pragma unroll
     for (int u = 0; u < BPT; ++u) {
       const int e = tid + u * DCN_THREADS;
-      uint32_t o = DCN_OOB;
+      uint32_t o = KAD_OOB;
       if (e < PIECES) {
         const int k = e / (NBC * 4), r = e - k * (NBC * 4), co = co0 + (r >> 2);
         if (co < cpad) o = (uint32_t)((((co * nchunk) * 9 + k) * 32 + (r & 3) * 8) * (int)sizeof(T));
@@ -534,7 +534,7 @@ __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom&
   __shared__ int s_box[4];
   __shared__ int s_reg[5];
 
-  // XCD-aware tile order, as dcn_block
+  // XCD-aware tile order over (image, tile) flattened, as the gathering kernel's
   const int q = (bx & 7) * (g.grid_x >> 3) + (bx >> 3);
   if (q >= a.n * g.tiles) return;  // whole block, before any barrier
   const int n = q / g.tiles, tile = q - n * g.tiles;
@@ -834,13 +834,8 @@ __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom&
     };
     auto blend = [&](int j, const frag (&c)[2][4], frag (&af)[2]) {
 #pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        Info16 in;
-        in.o01 = in.o23 = 0u;
-        in.w01 = r_w01[j][m];
-        in.w23 = r_w23[j][m];
-        af[m] = Ops::blend(c[m][0], c[m][1], c[m][2], c[m][3], in);
-      }
+      for (int m = 0; m < 2; ++m)
+        af[m] = Ops::blend(c[m][0], c[m][1], c[m][2], c[m][3], make_uint2(r_w01[j][m], r_w23[j][m]));
     };
     auto mma = [&](const frag (&af)[2], const frag (&bw)[NBF]) {
 #pragma unroll
@@ -899,14 +894,9 @@ __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom&
             if (ia & D2_SLOW) {
               const int cy0 = (int)((ia >> 14) & 0x7fffu), cx0 = (int)(ia & 0x3fffu);
               const int sx = (int)((ia >> 29) & 1u), sy = (int)((ia >> 30) & 1u);
-              const uint2 wv = s_iw[qi];
-              Info16 in;
-              in.o01 = in.o23 = 0u;
-              in.w01 = wv.x;
-              in.w23 = wv.y;
               const T* g0 = xb + ((int64_t)cy0 * a.w + cx0) * a.x_cs + ch;
               af[m] = Ops::blend(ld8<T>(g0), ld8<T>(g0 + sx * a.x_cs), ld8<T>(g0 + (int64_t)sy * a.w * a.x_cs),
-                                 ld8<T>(g0 + ((int64_t)sy * a.w + sx) * a.x_cs), in);
+                                 ld8<T>(g0 + ((int64_t)sy * a.w + sx) * a.x_cs), s_iw[qi]);
               any = true;
             }
           }
@@ -945,7 +935,7 @@ __device__ __forceinline__ void dsc2_block(const kad_dcn_args& a, const DcnGeom&
       pix_ok[m][i] = pl < npx && ty0 + oyl < g.ho && tx0 + pl - oyl * g.tw < g.wo;
     }
   float gsum[NBF];
-  auto epilogue = [&](auto act) {  // activation as a template argument, as in dcn_block
+  auto epilogue = [&](auto act) {  // activation as a template argument: no branch per value
     constexpr int ACT = decltype(act)::value;
 #pragma unroll
     for (int f = 0; f < NBF; ++f) {

@@ -15,8 +15,8 @@
 //    quad touches another line: 15 TB/s.
 //  * Loads run two k-steps ahead in registers, are blended, and enter LDS one k-step ahead; one
 //    barrier per k-step.  Taps are the outer loop: a tap's k-steps walk along the same corners' lines.
-//  * No input region is staged: samples may lie anywhere at one cost, a block needs about 55 KB of LDS
-//    and at most 128 registers, and two share a CU.  The kernel this one replaced staged the region a
+//  * No input region is staged: samples may lie anywhere at one cost, a block needs 48 to 55 KB of LDS (fp32
+//    with 96 columns 57, with 128 77: the epilogue's tile) and at most 128 registers, and two share a CU.  The kernel this one replaced staged the region a
 //    tile samples (147 KB, one block per CU; samples beyond it in a pass of their own) and read every
 //    weight fragment for 16 pixels only: it was bound by LDS reads and by its serial phases.
 //
@@ -45,11 +45,7 @@ template <typename T> struct DgOps {
     return make_uint2(pack_h2(w[0], w[1]), pack_h2(w[2], w[3]));
   }
   static __device__ __forceinline__ frag blend(const frag (&v)[4], const weights& w) {
-    Info16 in;
-    in.o01 = in.o23 = 0u;
-    in.w01 = w.x;
-    in.w23 = w.y;
-    return DcnFrag<T>::blend(v[0], v[1], v[2], v[3], in);
+    return DcnFrag<T>::blend(v[0], v[1], v[2], v[3], w);
   }
   static __device__ __forceinline__ floatx4 mma(const frag& a, const frag& b, floatx4 c) {
     return DcnFrag<T>::mma(a, b, c);
