@@ -3,8 +3,8 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--no-ops] [--no-cpu] [--no-kadcnet]
                     [--per-op-only] [--kadcnet-only]
 
-Step = one fused KADConv(256) forward on x [8, 256, 100, 100] fp16 (BASELINE
-config 2's metric shape), inputs resident in HBM, weights random from a seed
+Step = one fused KADConv(256) forward on x [8, 256, 100, 100] fp16 (a
+detector's neck map), inputs resident in HBM, weights random from a seed
 (synthetic; no checkpoint exists offline).  The forward is captured once in a
 HIP graph and replayed (the reference protocol, KAD-CNet/inference/benchmark_s.py:9-25):
 W warm-up replays, then 3 trials of K replays timed between events; the
@@ -15,12 +15,12 @@ Printed: one JSON line with
   roofline                 the dominant kernel (branch-0 DCN) timed alone with
                            events on its launch stream: algorithmic FLOPs / duration
                            against the fp16 dense MFMA peak;
-  forward_roofline         BASELINE's derived floor for the whole forward (10.33 us)
+  forward_roofline         the whole forward's bytes at 8 TB/s (10.33 us)
                            over the measured time;
   cpu_baseline             the oracle's fp32 CPU restatement of the reference forward
                            (plain PyTorch ops), same shape, on this host's cores;
   stages_us                per-stage event timings of one forward;
-  kadcnet_s_img_per_s      BASELINE config 5: KAD-CNet-S forward, batch 16, 800 x 800, fp16
+  kadcnet_s_img_per_s      KAD-CNet-S forward, batch 16, 800 x 800, fp16
                            (details and its CPU baseline under kadcnet_s);
   per_op                   configs 2-4 (DSC, KADDown, 1x1+SiLU, SE): GPU us, floor, and the
                            oracle's fp32 CPU us of the same workload;
@@ -127,7 +127,7 @@ KADCNET_DSC = [(12, 100), (10, 50), (10, 25), (16, 50), (16, 25), (16, 12), (22,
 
 
 def per_op_workloads():
-    """The other BASELINE configs as (name, launch, floor_us) with seeded inputs and weights."""
+    """The other workloads as (name, launch, floor_us) with seeded inputs and weights."""
     import kadconv
     from kadconv import synthetic as S
     out = []
@@ -230,7 +230,7 @@ PER_OP_BATCH = 10  # calls per graph for the amortised figure
 
 
 def per_op(steps, warmup, cpu=True):
-    """The other BASELINE configs, graph-timed (median of 3 trials, us per call) with
+    """The other workloads, graph-timed (median of 3 trials, us per call) with
     their floors, and the oracle's fp32 CPU time of the same workload.  `us` replays a graph
     of one call (the reference protocol); `us_graph10` replays a graph of PER_OP_BATCH calls
     of the same op on the same input and divides by PER_OP_BATCH: the replay's fixed cost (about
@@ -252,7 +252,7 @@ def per_op(steps, warmup, cpu=True):
 
 
 def config1(steps, warmup, cpu=True):
-    """BASELINE config 1: KADConv(64) and DSC(64) on [1, 64, 80, 80] fp32, every weight
+    """KADConv(64) and DSC(64) on [1, 64, 80, 80] fp32, every weight
     kaiming-uniform from seed 0.  Reported: the product's plain CPU forward (the
     plumbing the config asks for), the oracle's (the reference's plain path restated),
     and the fast HIP forward on the GPU for scale."""
@@ -319,7 +319,7 @@ def kadcnet_flops(hw=800):
 
 
 def kadcnet_s(iterations, warmup, cpu=True, batch=16, hw=800):
-    """the whole KAD-CNet-S forward (fused model, random init from
+    """The whole KAD-CNet-S forward (fused model, random init from
     seed 0, kadcnet.build_kadcnet_s), batch 16, 3 x 800 x 800 ~U[0, 1], fp16,
     model forward only (no NMS), HIP-graph replay, median of 3 trials
     (KAD-CNet/inference/benchmark_s.py:9-25).  CPU baseline: the oracle's fp32

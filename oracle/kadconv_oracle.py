@@ -191,7 +191,7 @@ def kadconv_forward(sd, x, n=3):
 
 
 # --------------------------------------------------------------------------- #
-# Fused blocks (BASELINE configs 4a/4b)
+# Fused blocks (1x1 + SiLU, SE)
 # --------------------------------------------------------------------------- #
 def conv1x1_silu(x, weight, bias):
     """KAD-CNet ``Conv`` after Conv-BN fusion with SiLU (models/common.py:43-57):

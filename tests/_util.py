@@ -1,4 +1,4 @@
-"""Shared helpers for the parity tests (tolerances stated in BASELINE.json north_star)."""
+"""Shared helpers for the parity tests, and their tolerances."""
 import torch
 
 FP32_REL = 1e-4      # fp32: max|d| <= 1e-4 * max|ref|

@@ -1,6 +1,6 @@
 """The product modules' plain forward on CPU (no GPU, no torchvision):
 kadconv.ops.deform_conv2d's CPU restatement and the KADConv / DSC modules built
-on it, against the oracle.  BASELINE config 1: KAD-Conv alone on the CPU
+on it, against the oracle.  KAD-Conv alone on the CPU
 plain-PyTorch path, x [1, 64, 80, 80] fp32 ~N(0, 1), every weight
 kaiming-uniform from seed 0 (conv_offset and LCSA included, so the offsets are
 not all zero).  Tolerance fp32: max|d| <= 1e-4 max|ref| (float64 oracle on the

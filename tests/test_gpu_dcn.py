@@ -91,7 +91,7 @@ def test_dcn_two_blocks_per_cu(dt, shape, pixel_major):
 @pytest.mark.parametrize('dt', ['f16', 'f32', 'bf16'])
 @pytest.mark.parametrize('C,H', [(128, 100), (256, 50), (512, 25)])
 def test_dcn_config2_shapes(dt, C, H):
-    """BASELINE config 2 scales, batch 8, offsets ~N(0, 2) px (with out-of-bounds samples)."""
+    """The three neck scales, batch 8, offsets ~N(0, 2) px (with out-of-bounds samples)."""
     dtype = DT[dt]
     x, off, mask, w, b = _inputs(8, C, C, H, H, seed=C)
     print(f'dcn_config2 dt={dt} C={C} H={H}', flush=True)

@@ -120,7 +120,7 @@ def test_dsc_two_blocks_per_cu(dt, shape, off_std, layout):
     check_close(got, _ref(x, ow, ob, w, b, mask, dtype), dtype, f'{dt} {shape} off_std={off_std}')
 
 
-# KAD-CNet-S at 800 x 800: the DSC(c, c) shapes of its 42 KADC4 layers,
+# KAD-CNet-S at 800 x 800 (batch 16): the DSC(c, c) shapes of its 42 KADC4 layers,
 # c in {12, 10, 10} at {100, 50, 25}^2, {16, 16, 16} at {50, 25, 12}^2, {22, 21, 21} at {25, 12, 6}^2
 KADCNET_DSC = [(12, 100), (10, 50), (10, 25), (16, 50), (16, 25), (16, 12), (22, 25), (21, 12), (21, 6)]
 

@@ -1,4 +1,4 @@
-"""KAD-CNet-S on the HIP kernels (BASELINE config 5) against the CPU oracle
+"""KAD-CNet-S on the HIP kernels against the CPU oracle
 (oracle/kadcnet_oracle.py), plus the network-level ops on their own.
 
 Network tolerances (stated here, measured on MI355X):
@@ -471,7 +471,7 @@ def _unexplained(kh, ko, ph, po, max_det=300):
 
 
 def test_kadcnet_config5_full_size():
-    """batch 16, 3 x 800 x 800 ~U[0, 1], fp16, fused model.  The batch runs on
+    """Batch 16, 3 x 800 x 800 ~U[0, 1], fp16, fused model.  The batch runs on
     the HIP plan; images 0 and 15 are checked against the float32 CPU oracle (every computation is
     per image).
 

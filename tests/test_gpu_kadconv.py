@@ -1,5 +1,5 @@
 """Parity of the fused HIP forwards (kadconv.enable_fast_inference, kadconv.ops,
-kadconv.blocks) against the CPU oracle, at the BASELINE configs.
+kadconv.blocks) against the CPU oracle, at the sizes of the benchmark.
 
 Weights are generated by state-dict name (oracle.make_*_state), loaded into
 the product modules, and the modules are cast to the run dtype; the oracle
@@ -165,7 +165,7 @@ def test_kadconv_metric_state(dt):
 @pytest.mark.parametrize('dt', ['f16', 'bf16', 'f32'])
 @pytest.mark.parametrize('C,H', [(128, 100), (256, 50), (512, 25)])
 def test_dsc_config2(dt, C, H):
-    """standalone DSC, batch 8, offsets ~N(0, 2) px."""
+    """Standalone DSC, batch 8, offsets ~N(0, 2) px."""
     import kadconv
     dtype = DT[dt]
     print(f'dsc dt={dt} C={C} H={H}', flush=True)
@@ -208,7 +208,7 @@ def test_dsc_f32_conv_offset_launch(layout, C, split):
 @pytest.mark.parametrize('dt,shape', [('f16', (16, 512, 50, 50)), ('f32', (2, 40, 9, 13)),
                                       ('bf16', (3, 72, 20, 21))])
 def test_conv1x1_silu(dt, shape):
-    """BASELINE config 4a: 1x1 conv + SiLU, W ~ N(0, 0.02)."""
+    """1x1 conv + SiLU, W ~ N(0, 0.02)."""
     import kadconv
     dtype = DT[dt]
     g = torch.Generator().manual_seed(7)
@@ -261,7 +261,7 @@ def test_conv1x1_shapes(dt, n, cin, cout, h, w, act, bias):
 
 @pytest.mark.parametrize('dt,shape', [('f16', (16, 1024, 25, 25)), ('f32', (2, 48, 7, 9)), ('bf16', (4, 96, 12, 12))])
 def test_squeeze_excitation(dt, shape):
-    """BASELINE config 4b: SE with reduction 16."""
+    """SE with reduction 16."""
     import kadconv
     dtype = DT[dt]
     C = shape[1]
@@ -374,7 +374,7 @@ def test_se_mlp_ws_matches_single_launch(n, c, hid, tiles):
 @pytest.mark.parametrize('dt,shape,c2', [('f16', (8, 256, 100, 100), 512), ('f32', (2, 24, 36, 44), 40),
                                          ('bf16', (1, 32, 27, 19), 16)])
 def test_kaddown(dt, shape, c2):
-    """BASELINE config 3 (builder-defined op, see oracle.kaddown_forward)."""
+    """KADDown (see oracle.kaddown_forward)."""
     import kadconv
     dtype = DT[dt]
     m = kadconv.KADDown(shape[1], c2)

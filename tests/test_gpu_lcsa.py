@@ -3,7 +3,7 @@ split variant) compared directly with sigmoid(oracle.lcsa_forward), i.e. the
 modulation mask of DSC.forward (KAD-Conv/kadconv/kad_conv.py:38-39,65), not
 through a DSC output where the DCN weights would damp a mask error.
 
-Shapes: BASELINE config 2's three DSC scales and the metric KADConv's three
+Shapes: the standalone DSC's three neck scales and the metric KADConv's three
 branch maps.  LCSA BatchNorm statistics are drawn far from identity (running
 mean in [-1, 1], variance in [0.3, 3], gamma in [0.5, 1.5], beta in [-0.5, 0.5])
 so that the folded BN is exercised.  The input is the dtype-rounded map; the
