@@ -34,6 +34,7 @@ from . import _ext
 GROUPED = True         # KADConvPlan: branch stages as grouped launches on one stream for small layers
 MAX_LISTS = 16         # KADConvPlan: input geometries whose recorded launches are kept
 GROUP_MAX_WORK = 1600  # ... whose full-resolution DSC has less work: N x tiles x column fragments
+GROUP_MAX_WORK_FEW, GROUP_FEW_TILES = 2048, 384  # ... or this much in fewer tiles
 
 
 def _f32(t):
@@ -262,12 +263,15 @@ class KADConvPlan:
         were measured to run one after another (KAD-CNet-S: 9.62 -> 9.14 ms per batch with
         every KADC4 grouped).  A heavy layer keeps the side streams: the coarse branches'
         DSCs and merges then fill the full-resolution DSC's last, partly empty round.
-        fp16 layers, grouped / streams (us; work): KADConv(256) [4, 75, 75] 122 / 132 (1.1k),
-        KADConv(192) [8, 80, 80] 103 / 102 (1.7k), KADConv(128) [8, 100, 100] 129 / 121 (1.9k),
-        KADConv(256) [16, 50, 50] 166 / 167 (1.9k), KADConv(256) [8, 100, 100] 180 / 167 (3.8k)."""
+        Grouped / streams, us a replay of a graph of one call (work; N x tiles): fp16 KADConv(256) [4, 75, 75]
+        128 / 148 (1.1k; 180), [16, 50, 50] 176 / 186 (1.9k; 320), bf16 218 / 226, fp32 353 / 359, [4, 100, 100]
+        fp16 131 / 141, fp32 325 / 329; but KADConv(128) [8, 100, 100] (1.9k; 640) bf16 176 / 168, fp32 265 / 256,
+        KADConv(192) [8, 80, 80] (1.6k; 400) fp16 111 / 119, fp32 234 / 227, KADConv(256) [5, 100, 100] (2.4k; 400)
+        bf16 199 / 190, [8, 100, 100] (3.8k; 640) fp16 193 / 191, in a graph of ten calls 176 / 165."""
         frags = min((self.branches[0].c + 15) // 16, 8)
-        work = x.shape[0] * _ext.dcn_tiles(x.shape[2], x.shape[3]) * frags
-        return self.groupable and work < GROUP_MAX_WORK
+        tiles = x.shape[0] * _ext.dcn_tiles(x.shape[2], x.shape[3])
+        limit = GROUP_MAX_WORK_FEW if tiles < GROUP_FEW_TILES else GROUP_MAX_WORK
+        return self.groupable and tiles * frags < limit
 
     def eligible(self, x):
         if not (x.is_cuda and x.dim() == 4 and x.dtype in (torch.float32, torch.float16, torch.bfloat16)):

@@ -3,6 +3,7 @@ are stubbed)."""
 import sys
 import threading
 
+import pytest
 import torch
 
 import kadconv
@@ -94,3 +95,13 @@ def test_lists_with_threads(monkeypatch):
         sys.setswitchinterval(every)
     assert not failed, failed[0]
     assert len(plan._lists) == fused.MAX_LISTS
+
+
+@pytest.mark.parametrize('dim,n,h,w,grouped', [
+    (256, 4, 75, 75, True), (256, 16, 50, 50, True), (256, 4, 100, 100, True),    # 1.1k; 1.9k in 320 tiles
+    (128, 8, 100, 100, False), (192, 8, 80, 80, False), (256, 5, 100, 100, False),
+    (256, 8, 100, 100, False), (32, 16, 100, 100, True)])
+def test_grouped_rule(dim, n, h, w, grouped):
+    """Which layers run as grouped launches: the full-resolution DSC's work and tiles."""
+    plan = KADConvPlan(kadconv.KADConv(dim).eval())
+    assert plan._grouped(torch.empty(n, dim, h, w, device='meta')) == grouped
