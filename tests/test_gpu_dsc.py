@@ -88,8 +88,7 @@ def test_dsc_small(dt, shape):
 @pytest.mark.parametrize('off_std', [0.6, 4.0])
 def test_dsc_branch0_shape(dt, off_std):
     """KADConv(256) branch 0 at the metric's spatial size (c = 86, 100 x 100),
-    NHWC out with a padded channel stride; off_std 4 px forces capped regions
-    and the global-memory sample pass."""
+    NHWC out with a padded channel stride; off_std 4 px samples far outside the tile."""
     dtype = DT[dt]
     x, ow, ob, w, b = _inputs(2, 86, 86, 100, 100, seed=86, off_std=off_std)
     mask = _mask(2, 100, 100, seed=86)
@@ -102,12 +101,13 @@ def test_dsc_branch0_shape(dt, off_std):
 @pytest.mark.parametrize('dt', ['f16', 'bf16'])
 @pytest.mark.parametrize('shape,off_std,layout', [((8, 10, 12, 100, 100), 2.0, 'nhwc'), ((12, 16, 16, 64, 64), 4.0, 'nchw'),
                                                   ((8, 22, 44, 80, 80), 2.0, 'nchw'), ((12, 3, 64, 60, 70), 1.0, 'nhwc'),
-                                                  ((6, 40, 33, 90, 90), 12.0, 'nhwc')])
+                                                  ((6, 40, 33, 90, 90), 12.0, 'nhwc'),
+                                                  ((6, 10, 15, 96, 100), 12.0, 'nchw'), ((24, 16, 16, 2, 1100), 12.0, 'nhwc')])
 def test_dsc_two_blocks_per_cu(dt, shape, off_std, layout):
-    """16-bit, stride 1, Cout <= 64 and >= 384 tile blocks: the launch runs on the
-    two-blocks-per-CU kernel.  Cin 3 / 10 / 22 / 40 (one half-chunk partly
-    padded, two, three), Cout not a multiple of 16, NCHW and NHWC outputs,
-    offsets up to 12 px (capped regions: samples from global memory)."""
+    """16-bit, stride 1, launches of >= 384 tile blocks: up to 16 input and output channels on the
+    narrow kernel (Cin 10 partly padded, offsets of 12 px: capped regions, samples from global
+    memory; wide thin tiles: two region buffers), the others on the gathering one (Cout not a
+    multiple of 16); NCHW and NHWC outputs."""
     from kadconv import _ext
     N, C, Co, H, W = shape
     assert N * _ext.dcn_tiles(H, W) >= 384
@@ -129,8 +129,8 @@ KADCNET_DSC = [(12, 100), (10, 50), (10, 25), (16, 50), (16, 25), (16, 12), (22,
 @pytest.mark.parametrize('C,H', KADCNET_DSC)
 def test_dsc_kadcnet_shapes(dt, C, H):
     """Every small-channel DSC shape of KAD-CNet-S, batch 16, channels-last output (the
-    network's layout), offsets ~N(0, 2) px: the fp16 launches with >= 384 tile blocks run on
-    the two-blocks-per-CU kernel, the others on the general one."""
+    network's layout), offsets ~N(0, 2) px: fp16 up to 16 channels runs on the narrow kernel, the
+    others on the gathering one."""
     dtype = DT[dt]
     x, ow, ob, w, b = _inputs(16, C, C, H, H, seed=C * 7 + H)
     mask = _mask(16, H, H, seed=C + H)
@@ -141,10 +141,11 @@ def test_dsc_kadcnet_shapes(dt, C, H):
 
 
 @pytest.mark.parametrize('dt', ['f16', 'bf16'])
-def test_dsc_two_blocks_per_cu_gap(dt):
-    """GAP partials of the two-blocks-per-CU kernel: fp32 sums of the rounded outputs."""
+@pytest.mark.parametrize('Co', [16, 20])
+def test_dsc_two_blocks_per_cu_gap(dt, Co):
+    """GAP partials of the narrow kernel (Cout 16) and the gathering one: fp32 sums of the rounded outputs."""
     from kadconv import _ext
-    N, C, Co, H, W = 8, 16, 20, 100, 100
+    N, C, H, W = 8, 16, 100, 100
     assert N * _ext.dcn_tiles(H, W) >= 384
     x, ow, ob, w, b = _inputs(N, C, Co, H, W, seed=5)
     mask = _mask(N, H, W, seed=5)
@@ -188,9 +189,7 @@ def test_dsc_gap_partials_sum_to_mean(dt):
 
 @pytest.mark.parametrize('dt', ['f16', 'bf16'])
 def test_dsc_far_offsets(dt):
-    """Offsets of ~20 px: most samples fall outside any region that fits the
-    LDS budget (capped or 1 x 1 regions), so the pass from global memory
-    carries them; many are dead (outside the image)."""
+    """Offsets of ~20 px: most samples lie far from their tile, many are dead (outside the image)."""
     dtype = DT[dt]
     x, ow, ob, w, b = _inputs(2, 40, 48, 37, 41, seed=20, off_std=20.0)
     mask = _mask(2, 37, 41, seed=20)

@@ -76,6 +76,14 @@ def test_narrow_outputs(dt, mode, shape):
     test_gather_edges(dt, mode, shape, 1, 2.0)
 
 
+@pytest.mark.parametrize('dt', ['f16', 'bf16'])
+@pytest.mark.parametrize('shape', [(2, 12, 16, 60, 64), (1, 40, 15, 64, 70), (1, 144, 16, 48, 61)])
+def test_narrow_outputs_far_offsets(dt, shape):
+    """The narrow kernel with offsets from memory, one, three and nine half-chunks, samples beyond the
+    region that a tile stages."""
+    test_gather_edges(dt, 'dcn', shape, 1, 12.0)
+
+
 @pytest.mark.parametrize('c,hid', [(10, 32), (16, 16), (40, 40), (86, 86), (90, 91), (128, 128), (85, 7)])
 def test_se_tail_sizes(c, hid):
     """Fused squeeze-excitation with weights that fit the LDS beside the partials and ones that do not
