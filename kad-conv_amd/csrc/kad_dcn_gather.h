@@ -20,11 +20,11 @@
 //    tile samples (147 KB, one block per CU; samples beyond it in a pass of their own) and read every
 //    weight fragment for 16 pixels only: it was bound by LDS reads and by its serial phases.
 //
-// Measured (fp16, alone, 10 launches in a graph; this kernel / the replaced one): [8, 128, 100, 100] DSC
-// 75 / 105 us, branch 0 of KADConv(256) at 100 x 100 (86 channels) 65 / 84 us; fp32 [4, 128, 100, 100]
-// DSC 219 / 417 us.  A block of 86 channels takes 34k cycles for its 27 k-steps when two share the CU
-// (620 per k-step and block; the loads alone take about 600 through L1's 64 B / clk) and 27k alone, and
-// some 30k for conv_offset, records, epilogue and squeeze-excitation.
+// Measured (alone, 10 launches in a graph; this kernel / the replaced one, us): fp16 [8, 128, 100, 100] DSC
+// 77 / 105, branch 0 of KADConv(256) at 100 x 100 (86 channels) 58 / 84; fp32 [4, 128, 100, 100] DSC 204 / 417.
+// By clock64 stamps a block of 86 channels takes 34k cycles for its 27 k-steps when two share the CU (620 per
+// k-step and block; the loads alone take about 600 through L1's 64 B / clk) and 27k alone, and some 30k for
+// conv_offset, records, epilogue and squeeze-excitation.
 #pragma once
 #include <type_traits>
 
