@@ -16,9 +16,10 @@
 //  * Loads run two k-steps ahead in registers, are blended, and enter LDS one k-step ahead; one
 //    barrier per k-step.  Taps are the outer loop: a tap's k-steps walk along the same corners' lines.
 //  * No input region is staged: samples may lie anywhere at one cost, a block needs 48 to 55 KB of LDS (fp32
-//    with 96 columns 57, with 128 77: the epilogue's tile) and at most 128 registers, and two share a CU.  The kernel this one replaced staged the region a
-//    tile samples (147 KB, one block per CU; samples beyond it in a pass of their own) and read every
-//    weight fragment for 16 pixels only: it was bound by LDS reads and by its serial phases.
+//    with 96 columns 57, with 128 77: the epilogue's tile) and at most 128 registers, and two share a CU.
+//    The kernel this one replaced staged the region a tile samples (147 KB, one block per CU; samples beyond
+//    it in a pass of their own) and read every weight fragment for 16 pixels only: it was bound by LDS reads
+//    and by its serial phases.
 //
 // Measured (alone, 10 launches in a graph; this kernel / the replaced one, us): fp16 [8, 128, 100, 100] DSC
 // 77 / 105, branch 0 of KADConv(256) at 100 x 100 (86 channels) 58 / 84; fp32 [4, 128, 100, 100] DSC 204 / 417.
@@ -547,6 +548,9 @@ static int dg_launch(const kad_dcn_args& a, const DcnGeom& g, int mode, hipStrea
   return check_launch(mode == MODE_FUSED ? "kad_dsc_fwd" : "kad_dcn_fwd");
 }
 
+// Columns by Cout alone: 16, 32, 64, 96 or blocks of 128.  The padding of 33 .. 48 channels to 64 columns and of
+// 65 .. 80 to 96 costs less than a form of 48 or 80 would gain: the replaced kernel had those, and DSC took (us,
+// it / this) 48 channels fp16 [8, 50, 50] 40 / 35, bf16 48 / 43, fp32 82 / 62; 80 channels 51 / 44, 71 / 59, 150 / 104.
 template <typename T> int dcn_gather(const kad_dcn_args& a, const DcnGeom& g, int mode, hipStream_t st) {
   if (a.cout <= 16) return dg_launch<T, 1>(a, g, mode, st);
   switch (ceil_div(a.cout, 32)) {
